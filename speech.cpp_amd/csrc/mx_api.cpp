@@ -25,6 +25,9 @@ struct mx_backend {
     void *scratch = nullptr;         // grows on demand outside graph capture
     size_t scratch_size = 0;
     uint64_t scratch_gen = 0;        // counts scratch reallocations: a graph recorded before one holds a freed address
+    void *work = nullptr;            // ensure_work's buffer, and those it replaced (freed with the backend)
+    size_t work_size = 0;
+    std::vector<void *> old_work;
     uint8_t *staging = nullptr;      // device staging for ggml-layout uploads and downloads
     size_t staging_size = 0;
     bool capturing = false;
@@ -220,6 +223,27 @@ int ensure_scratch(mx_backend *be, size_t bytes) {
     return MX_SUCCESS;
 }
 
+// Scratch for an op that has a path without any: false (and nothing changed) where the stream is being recorded and
+// the buffer would have to grow, or the device has no memory left for it; the op then takes that path. A buffer that
+// grew is kept until the backend goes: graphs recorded on it, by mx_graph_begin or by the caller on the backend's
+// stream, stay valid. Sizes at least double, so what is kept is less than the buffer in use.
+bool ensure_work(mx_backend *be, size_t bytes) {
+    if (bytes <= be->work_size) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (be->capturing || hipStreamIsCapturing(be->stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
+        return false;
+    const size_t size = std::max<size_t>(mx::align_up(bytes, 1 << 20), 2 * be->work_size);
+    void *p = nullptr;
+    if (hipMalloc(&p, size) != hipSuccess) {
+        (void)hipGetLastError();  // the failure is handled here: no later launch check should meet it
+        return false;
+    }
+    if (be->work) be->old_work.push_back(be->work);
+    be->work = p;
+    be->work_size = size;
+    return true;
+}
+
 int ensure_staging(mx_backend *be) {
     if (be->staging) return MX_SUCCESS;
     HIP_OK(hipMalloc(&be->staging, kStagingPiece), "allocate staging");
@@ -287,6 +311,8 @@ MX_API void mx_backend_free(mx_backend *be) {
     (void)hipSetDevice(be->device);
     if (be->stream) (void)hipStreamSynchronize(be->stream);
     if (be->scratch) (void)hipFree(be->scratch);
+    if (be->work) (void)hipFree(be->work);
+    for (void *p : be->old_work) (void)hipFree(p);
     if (be->staging) (void)hipFree(be->staging);
     if (be->err) (void)hipFree(be->err);
     if (be->stream) (void)hipStreamDestroy(be->stream);
@@ -781,6 +807,36 @@ static int gemm_dq_group(mx_backend *be, int n, const mx_tensor *const *src0, co
     return MX_SUCCESS;
 }
 
+// M > 8 on F16 / F32 weights: per batch slice, one launch over every weight sharing src1 (behind the pass that rounds
+// src1 to fp16 for F16 weights on the larger tiles). *done stays false where the product needs scratch that cannot be
+// had now: the mat-vec over groups of columns computes it without any.
+static int gemm_f_group(mx_backend *be, int n, const mx_tensor *const *src0, const mx_tensor *src1,
+                        const mx_tensor *const *dst, bool *done) {
+    const mx_tensor *w0 = src0[0];
+    const int64_t K = w0->ne[0], M = src1->ne[1];
+    int64_t N[4], ldy[4];
+    for (int i = 0; i < n; i++) {
+        N[i] = src0[i]->ne[1];
+        ldy[i] = (int64_t)(dst[i]->nb[1] / 4);
+    }
+    if (!ensure_work(be, mx::gemm_f_scratch_bytes(w0->type, n, N, M, K))) return MX_SUCCESS;
+    *done = true;
+    const int64_t r2 = src1->ne[2] / w0->ne[2], r3 = src1->ne[3] / w0->ne[3];
+    for (int64_t i13 = 0; i13 < src1->ne[3]; i13++)
+        for (int64_t i12 = 0; i12 < src1->ne[2]; i12++) {
+            const float *x = (const float *)((const uint8_t *)src1->data + i12 * src1->nb[2] + i13 * src1->nb[3]);
+            const void *w[4];
+            float *y[4];
+            for (int i = 0; i < n; i++) {
+                w[i] = (const uint8_t *)src0[i]->data + (i12 / r2) * src0[i]->nb[2] + (i13 / r3) * src0[i]->nb[3];
+                y[i] = (float *)((uint8_t *)dst[i]->data + i12 * dst[i]->nb[2] + i13 * dst[i]->nb[3]);
+            }
+            HIP_OK(mx::launch_gemm_f(w0->type, n, w, N, x, (int64_t)src1->nb[1], y, ldy, M, K, be->work, be->stream),
+                   "GEMM launch");
+        }
+    return MX_SUCCESS;
+}
+
 // Products sharing src1: n problems (n <= 4) of the same type and K, each with its own rows and dst; `f` (validated
 // by mx_mul_mat_fused, mat-vec path only) fuses the neighbouring norm / SwiGLU / residual ADD.
 static int matvec_group(mx_backend *be, int n, const mx_tensor *const *src0, const mx_tensor *src1,
@@ -828,6 +884,11 @@ static int matvec_group(mx_backend *be, int n, const mx_tensor *const *src0, con
         if (fits && mx::gemm_dq_supported(a.type, M, a.K)) return gemm_dq_group(be, n, src0, src1, dst);
         if (a.type == MX_TYPE_Q4_K && a.K % 256 == 0) return gemm_q4k_group(be, n, src0, src1, dst);
         if (mx::gemm_kq_supported(a.type, a.K)) return gemm_kq_group(be, n, src0, src1, dst);
+        if (mx::gemm_f_supported(a.type, M, a.K, (int64_t)src1->nb[1])) {
+            bool done = false;
+            const int rc = gemm_f_group(be, n, src0, src1, dst, &done);
+            if (rc || done) return rc;
+        }
     }
     const int ncmax = max_cols(a.type, a.K);
     for (int64_t m0 = 0; m0 < M; m0 += ncmax) {
