@@ -112,8 +112,7 @@ __device__ __forceinline__ void fused_prologue(const MatvecArgs &a, const float 
                 const float4 v = piece(c, base, load_x4(x + c * a.x_col_stride, base + 4 * tid, K));
                 ss += (double)(v.x * v.x) + (double)(v.y * v.y) + (double)(v.z * v.z) + (double)(v.w * v.w);
             }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+            ss = wave_sum_d(ss);
             if (lane == 0) red[c][wave] = ss;
         }
         __syncthreads();

@@ -53,6 +53,66 @@ __device__ __forceinline__ float sum_lanes(float v) {
     return v;
 }
 
+// The butterfly x_i + x_(i ^ 32), then ^ 16, 8, 4, 2, 1, in every lane, without an LDS round trip: the halves and the rows
+// of 16 are exchanged by permlane swaps; after the step over 8 the values repeat every 8 lanes (then every 4), so that
+// rotations of a row by 8 and 4 read lanes i ^ 8 and one equal to lane i ^ 4.
+namespace lanes {
+constexpr int ROR8 = 0x128, ROR4 = 0x124;
+__device__ __forceinline__ void swap32(uint32_t v, uint32_t &lo, uint32_t &hi) {  // both halves' values in every lane
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    lo = r[0];
+    hi = r[1];
+}
+__device__ __forceinline__ void swap16(uint32_t v, uint32_t &lo, uint32_t &hi) {  // both rows' of a pair of rows
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    lo = r[0];
+    hi = r[1];
+}
+}  // namespace lanes
+
+__device__ __forceinline__ double wave_sum_d(double v) {
+    auto w = [](double x, int i) { return (uint32_t)(__builtin_bit_cast(uint64_t, x) >> (32 * i)); };
+    auto d = [](uint32_t lo, uint32_t hi) { return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo); };
+    uint32_t a0, b0, a1, b1;
+    lanes::swap32(w(v, 0), a0, b0);
+    lanes::swap32(w(v, 1), a1, b1);
+    v = d(a0, a1) + d(b0, b1);
+    lanes::swap16(w(v, 0), a0, b0);
+    lanes::swap16(w(v, 1), a1, b1);
+    v = d(a0, a1) + d(b0, b1);
+#define MX_STEP(CTRL) v += d((uint32_t)dpp_i<CTRL>(0, (int)w(v, 0)), (uint32_t)dpp_i<CTRL>(0, (int)w(v, 1)))
+    MX_STEP(lanes::ROR8);
+    MX_STEP(lanes::ROR4);
+    MX_STEP(dpp::XOR2);
+    MX_STEP(dpp::XOR1);
+#undef MX_STEP
+    return v;
+}
+__device__ __forceinline__ float wave_sum_f(float v) {
+    uint32_t a, b;
+    lanes::swap32(__float_as_uint(v), a, b);
+    v = __uint_as_float(a) + __uint_as_float(b);
+    lanes::swap16(__float_as_uint(v), a, b);
+    v = __uint_as_float(a) + __uint_as_float(b);
+    v += dpp_f<lanes::ROR8>(0.0f, v);
+    v += dpp_f<lanes::ROR4>(0.0f, v);
+    v += dpp_f<dpp::XOR2>(0.0f, v);
+    v += dpp_f<dpp::XOR1>(0.0f, v);
+    return v;
+}
+__device__ __forceinline__ float wave_max_f(float v) {
+    uint32_t a, b;
+    lanes::swap32(__float_as_uint(v), a, b);
+    v = fmaxf(__uint_as_float(a), __uint_as_float(b));
+    lanes::swap16(__float_as_uint(v), a, b);
+    v = fmaxf(__uint_as_float(a), __uint_as_float(b));
+    v = fmaxf(v, dpp_f<lanes::ROR8>(0.0f, v));
+    v = fmaxf(v, dpp_f<lanes::ROR4>(0.0f, v));
+    v = fmaxf(v, dpp_f<dpp::XOR2>(0.0f, v));
+    v = fmaxf(v, dpp_f<dpp::XOR1>(0.0f, v));
+    return v;
+}
+
 // ------------------------------------------------------------------------------------------------------------------
 // Buffer-to-LDS copies and their waits (the prefill GEMMs' and the MoE product's operand rings).
 // ------------------------------------------------------------------------------------------------------------------
