@@ -1252,9 +1252,10 @@ MX_API int mx_supports_flash_attn_ext(const mx_tensor *q, const mx_tensor *k, co
            dst->ne[3] == 1 && contiguous(dst) && dst->data && q->ne[1] <= 65535 && q->ne[2] <= 65535;
 }
 
-// Validation, arguments and scratch of an attention launch (mx_flash_attn_ext; mx_attn_decode).
+// Validation, arguments and scratch of an attention launch (mx_flash_attn_ext; mx_attn_decode). *mfma (when given)
+// becomes true for a call that goes to the matrix cores: several rows, and the scratch of its splits can be had.
 static int fa_args(mx_backend *be, const mx_tensor *q, const mx_tensor *k, const mx_tensor *v, const mx_tensor *mask,
-                   const mx_tensor *dst, float scale, mx::FaArgs *a) {
+                   const mx_tensor *dst, float scale, mx::FaArgs *a, bool *mfma = nullptr) {
     if (!mx_supports_flash_attn_ext(q, k, v, mask, dst, 0.0f, 0.0f))
         return fail(MX_UNSUPPORTED, "FLASH_ATTN_EXT: unsupported tensors");
     a->q = (const float *)q->data;
@@ -1275,11 +1276,21 @@ static int fa_args(mx_backend *be, const mx_tensor *q, const mx_tensor *k, const
     a->v_nb2 = (int64_t)v->nb[2];
     a->m_nb1 = mask ? (int64_t)mask->nb[1] : 0;
     a->scale = scale;
+    auto part_bytes = [&]() {
+        return (size_t)a->n_q * (size_t)a->n_head * (size_t)a->nsplit * (size_t)(a->D + 2) * 4;
+    };
+    if (mfma && mx::fa_mfma_supported(*a)) {
+        mx::fa_mfma_split(*a);
+        if (a->nsplit == 1 || ensure_work(be, part_bytes())) {
+            a->part = (float *)be->work;
+            *mfma = true;
+            return MX_SUCCESS;
+        }
+    }
     a->nsplit = mx::fa_splits(a->n_q, a->n_head, a->n_kv, a->gqa, a->D);
     a->split_len = ((a->n_kv + 63) / 64 + a->nsplit - 1) / a->nsplit * 64;  // whole 64-position blocks per split
     if (a->nsplit > 1) {
-        const size_t need = (size_t)a->n_q * (size_t)a->n_head * (size_t)a->nsplit * (size_t)(a->D + 2) * 4;
-        int rc = ensure_scratch(be, need);
+        int rc = ensure_scratch(be, part_bytes());
         if (rc) return rc;
         a->part = (float *)be->scratch;
     }
@@ -1291,8 +1302,9 @@ MX_API int mx_flash_attn_ext(mx_backend *be, const mx_tensor *q, const mx_tensor
     int rc = check_be(be);
     if (rc) return rc;
     mx::FaArgs a{};
-    if ((rc = fa_args(be, q, k, v, mask, dst, scale, &a))) return rc;
-    HIP_OK(mx::launch_flash_attn(a, be->stream), "FLASH_ATTN_EXT launch");
+    bool mfma = false;
+    if ((rc = fa_args(be, q, k, v, mask, dst, scale, &a, &mfma))) return rc;
+    HIP_OK(mfma ? mx::launch_fa_mfma(a, be->stream) : mx::launch_flash_attn(a, be->stream), "FLASH_ATTN_EXT launch");
     return MX_SUCCESS;
 }
 

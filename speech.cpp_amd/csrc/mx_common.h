@@ -340,6 +340,13 @@ struct QkvPostArgs {
 };
 hipError_t launch_qkv_post(const QkvPostArgs &a, int64_t rows, hipStream_t s);
 hipError_t launch_flash_attn(const FaArgs &a, hipStream_t s);
+// The merge of a.nsplit > 1 splits' partials into dst (k_fa_merge).
+hipError_t launch_fa_merge(const FaArgs &a, hipStream_t s);
+// Several query rows on the matrix cores (attn.hip): whether it takes the call, the splits it takes (a.nsplit,
+// a.split_len; nsplit > 1 needs a.part as above), the launch.
+bool fa_mfma_supported(const FaArgs &a);
+void fa_mfma_split(FaArgs &a);
+hipError_t launch_fa_mfma(const FaArgs &a, hipStream_t s);
 // One decode row: launch_qkv_post and launch_flash_attn in one attention launch (head size 128, gqa 1, 2 or 4; the
 // attention reads the caches pa stores into).
 hipError_t launch_attn_decode(const FaArgs &a, const QkvPostArgs &pa, hipStream_t s);
