@@ -16,11 +16,27 @@ __device__ __forceinline__ MatvecProblem pick_problem(const MatvecArgs &a, int i
     return i == 0 ? a.prob[0] : (i == 1 ? a.prob[1] : (i == 2 ? a.prob[2] : a.prob[3]));
 }
 
-// float4s of each activation column every thread loads ahead of the weights (elements 1024 i + 4 tid, i < XPRE).
+// The most threads of a workgroup. Every workgroup quantizes all of its columns, so the more there are the more rows
+// should share that: eight waves from two columns on (four waves: 2048 + 1024 + 1024 Q8_0 rows of K = 2048, five columns
+// behind a norm, 12.0 us; eight 7.7; Q6_K, 2048 rows of K = 6144, eight columns 26.7 and 17.2). Q5_K keeps four: its dots
+// take more registers than eight waves leave. mv_fixed: launch_nc always takes that many.
+template <int TYPE, int NC>
+__host__ __device__ constexpr int mv_threads() { return NC >= 2 && TYPE != MX_TYPE_Q5_K ? 512 : 256; }
+template <int TYPE, int NC>
+__host__ __device__ constexpr bool mv_fixed() { return NC == 1 || TYPE == MX_TYPE_Q8_0 || TYPE == MX_TYPE_Q5_K; }
+// ... and whether a workgroup goes on to further rows with the columns it has quantized.
+template <int NC>
+__host__ __device__ constexpr bool mv_loops() { return NC >= 2; }
+// A workgroup's waves; the elements of a column it handles at once are 256 a wave (a float4 a thread). Below, the float4s
+// of each column every thread loads ahead of the weights (elements PIECE i + 4 tid, i < XPRE).
+template <int TYPE, int NC>
+__device__ __forceinline__ int mv_waves() {
+    return mv_fixed<TYPE, NC>() ? mv_threads<TYPE, NC>() / 64 : (int)blockDim.x / 64;
+}
 template <int NC>
 __host__ __device__ constexpr int xpre() { return NC == 1 ? 4 : (NC == 2 ? 2 : 1); }
 
-// Quantizes the 1024-element piece at `base` of one activation column (v = elements base + 4 tid .. + 3) into LDS:
+// Quantizes one piece, at `base`, of one activation column (v = elements base + 4 tid .. + 3) into LDS:
 // Q8_0 weights take 32-blocks (d rounded to fp16 and back, as the CPU dot reads it), K-quants Q8_K 256-blocks with
 // their 16-element sums (Q4_K: quants in unit order and sums of 32, as its dot reads them). Every wave of the
 // workgroup calls it with the same `base`.
@@ -63,16 +79,18 @@ __device__ __forceinline__ float4 load_x4(const float *xc, int e, int K) {
 // The fused prologue: each column x becomes silu(x) * glu_b (ggml_vec_swiglu_f32's scalar form) when glu_b is set,
 // then mul(rms_norm(x, eps), norm_w) when norm_w is set -- the squares (rounded to float) summed in double over the
 // workgroup, the mean rounded to float, x * (1 / sqrtf(mean + eps)) then times the weight, as the separate ops round
-// -- and is quantized. Pieces of 1024 elements past the preloaded ones are read again after the sum.
+// -- and is quantized. Pieces past the preloaded ones are read again after the sum.
 template <int TYPE, int NC>
 __device__ __forceinline__ void fused_prologue(const MatvecArgs &a, const float *x, int xi12, int i13,
                                                float4 (&xr)[NC][xpre<NC>()], const float4 (&br)[NC][xpre<NC>()],
                                                const float4 (&wr)[xpre<NC>()], int8_t *xq, float *xd, int *xbs) {
     constexpr int XP = xpre<NC>();
+    const int PIECE = 256 * mv_waves<TYPE, NC>();
     constexpr int XDB = TYPE == MX_TYPE_Q8_0 ? 32 : 256;
     const int K = (int)a.K;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    __shared__ double red[NC][4];
+    constexpr int MW = mv_threads<TYPE, NC>() / 64;
+    __shared__ double red[NC][MW];
     const float *gb = a.glu_b ? a.glu_b + xi12 * a.x_b2 + i13 * a.x_b3 : nullptr;
     // glu of one loaded piece; the preloaded pieces' second operands came in with x (br)
     auto piece_b = [&](float4 v, float4 b) -> float4 {
@@ -82,15 +100,19 @@ __device__ __forceinline__ void fused_prologue(const MatvecArgs &a, const float 
         v.w = v.w / (1.0f + expf(-v.w)) * b.w;
         return v;
     };
-    auto piece = [&](int c, int base, float4 v) -> float4 {
+    // Every column's elements of the piece at `base`, past the preloaded ones: all of their loads go out before
+    // the first is used. (Column after column, a product of several columns waited for K / PIECE - 1 loads of each in a
+    // row.)
+    auto piece = [&](int base, float4 (&v)[NC]) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) v[c] = load_x4(x + c * a.x_col_stride, base + 4 * tid, K);
         if (gb) {
-            const float4 b = load_x4(gb + c * a.x_col_stride, base + 4 * tid, K);
-            v.x = v.x / (1.0f + expf(-v.x)) * b.x;
-            v.y = v.y / (1.0f + expf(-v.y)) * b.y;
-            v.z = v.z / (1.0f + expf(-v.z)) * b.z;
-            v.w = v.w / (1.0f + expf(-v.w)) * b.w;
+            float4 b[NC];
+#pragma unroll
+            for (int c = 0; c < NC; c++) b[c] = load_x4(gb + c * a.x_col_stride, base + 4 * tid, K);
+#pragma unroll
+            for (int c = 0; c < NC; c++) v[c] = piece_b(v[c], b[c]);
         }
-        return v;
     };
     if (gb) {
 #pragma unroll
@@ -100,32 +122,41 @@ __device__ __forceinline__ void fused_prologue(const MatvecArgs &a, const float 
     }
     float scale[NC];
     if (a.norm_w) {
+        auto square = [](float4 v) {
+            return (double)(v.x * v.x) + (double)(v.y * v.y) + (double)(v.z * v.z) + (double)(v.w * v.w);
+        };
+        double ss[NC];
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            double ss = 0.0;
+            ss[c] = 0.0;
 #pragma unroll
-            for (int i = 0; i < XP; i++) {
-                const float4 v = xr[c][i];  // zero past K
-                ss += (double)(v.x * v.x) + (double)(v.y * v.y) + (double)(v.z * v.z) + (double)(v.w * v.w);
-            }
-            for (int base = 1024 * XP; base < K; base += 1024) {
-                const float4 v = piece(c, base, load_x4(x + c * a.x_col_stride, base + 4 * tid, K));
-                ss += (double)(v.x * v.x) + (double)(v.y * v.y) + (double)(v.z * v.z) + (double)(v.w * v.w);
-            }
-            ss = wave_sum_d(ss);
-            if (lane == 0) red[c][wave] = ss;
+            for (int i = 0; i < XP; i++) ss[c] += square(xr[c][i]);  // zero past K
+        }
+        for (int base = PIECE * XP; base < K; base += PIECE) {
+            float4 v[NC];
+            piece(base, v);
+#pragma unroll
+            for (int c = 0; c < NC; c++) ss[c] += square(v[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            ss[c] = wave_sum_d(ss[c]);
+            if (lane == 0) red[c][wave] = ss[c];
+            if (!mv_fixed<TYPE, NC>() && lane == 0 && PIECE < 256 * MW) red[c][MW / 2 + wave] = 0.0;  // four waves of eight
         }
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const double tot = red[c][0] + red[c][1] + red[c][2] + red[c][3];
+            double tot = red[c][0];
+#pragma unroll
+            for (int w = 1; w < MW; w++) tot += red[c][w];
             const float mean = (float)(tot / (double)K);
             scale[c] = 1.0f / sqrtf(mean + a.norm_eps);
         }
     }
-    auto normed = [&](int c, int base, float4 v) -> float4 {
+    auto normed = [&](int c, int base, int i, float4 v) -> float4 {  // i: the preloaded piece, or -1
         if (a.norm_w) {
-            const float4 w = base < 1024 * XP ? wr[base / 1024] : load_x4(a.norm_w, base + 4 * tid, K);
+            const float4 w = i >= 0 ? wr[i] : load_x4(a.norm_w, base + 4 * tid, K);
             v.x = (v.x * scale[c]) * w.x;
             v.y = (v.y * scale[c]) * w.y;
             v.z = (v.z * scale[c]) * w.z;
@@ -133,25 +164,55 @@ __device__ __forceinline__ void fused_prologue(const MatvecArgs &a, const float 
         }
         return v;
     };
+    auto quantize = [&](int c, int base, int i, float4 v) {
+        quantize_piece<TYPE>(normed(c, base, i, v), base, K, a.rounding, xq + c * K, xd + c * (K / XDB),
+                             xbs + c * xbs_per_col<TYPE>(K));
+    };
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-        const float *xc = x + c * a.x_col_stride;
+    for (int c = 0; c < NC; c++)
 #pragma unroll
         for (int i = 0; i < XP; i++)
-            if (1024 * i < K)
-                quantize_piece<TYPE>(normed(c, 1024 * i, xr[c][i]), 1024 * i, K, a.rounding, xq + c * K,
-                                     xd + c * (K / XDB), xbs + c * xbs_per_col<TYPE>(K));
-        for (int base = 1024 * XP; base < K; base += 1024)
-            quantize_piece<TYPE>(normed(c, base, piece(c, base, load_x4(xc, base + 4 * tid, K))), base, K, a.rounding,
-                                 xq + c * K, xd + c * (K / XDB), xbs + c * xbs_per_col<TYPE>(K));
+            if (PIECE * i < K) quantize(c, PIECE * i, i, xr[c][i]);
+    for (int base = PIECE * XP; base < K; base += PIECE) {
+        float4 v[NC];
+        piece(base, v);
+#pragma unroll
+        for (int c = 0; c < NC; c++) quantize(c, base, -1, v[c]);
+    }
+}
+
+// The plain prologue: every column quantized into LDS, the preloaded pieces first, the others piece by piece with all
+// columns' loads in flight.
+template <int TYPE, int NC>
+__device__ __forceinline__ void plain_prologue(const MatvecArgs &a, const float *x, const float4 (&xr)[NC][xpre<NC>()],
+                                               int8_t *xq, float *xd, int *xbs) {
+    constexpr int XP = xpre<NC>();
+    const int PIECE = 256 * mv_waves<TYPE, NC>();
+    constexpr int XDB = TYPE == MX_TYPE_Q8_0 ? 32 : 256;
+    const int K = (int)a.K;
+    auto quantize = [&](int c, int base, float4 v) {
+        quantize_piece<TYPE>(v, base, K, a.rounding, xq + c * K, xd + c * (K / XDB), xbs + c * xbs_per_col<TYPE>(K));
+    };
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int i = 0; i < XP; i++)
+            if (PIECE * i < K) quantize(c, PIECE * i, xr[c][i]);
+    for (int base = PIECE * XP; base < K; base += PIECE) {
+        float4 v[NC];
+#pragma unroll
+        for (int c = 0; c < NC; c++) v[c] = load_x4(x + c * a.x_col_stride, base + 4 * (int)threadIdx.x, K);
+#pragma unroll
+        for (int c = 0; c < NC; c++) quantize(c, base, v[c]);
     }
 }
 
 // FUSED: the instantiation that reads the fused operands (norm weight, SwiGLU input, residual); the plain one is
 // compiled without them, so products with no fusion keep their smaller register footprint.
 template <int TYPE, int NC, int LPR, bool FUSED>
-__global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
+__global__ __launch_bounds__((mv_threads<TYPE, NC>())) void k_matvec(MatvecArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
+    const int NW = mv_waves<TYPE, NC>();
     const int K = (int)a.K;
     const int tid = threadIdx.x;
     // The argument block's fields on the way to the first weight load, requested together into scalar registers:
@@ -169,6 +230,8 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
         if constexpr (TYPE == MX_TYPE_Q5_K || TYPE == MX_TYPE_Q6_K) asm volatile("" ::"s"(p.w.p3));
         if constexpr (FUSED) asm volatile("" ::"s"(a.glu_b), "s"(a.norm_w), "s"(p.res));
     }
+    // a narrower problem of a group: the grid is the widest one's
+    if ((int64_t)blockIdx.x * (NW * (64 / LPR)) >= p.N) return;
     // Batch slice; a single slice (decode) takes no division.
     int i12 = 0, i13 = 0, mat = 0;
     if (a.nbatch > 1) {
@@ -191,11 +254,12 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
     // The activation loads go first: x -> quantization -> LDS is the prologue's critical path, and the memory counter
     // retires loads in order, so waiting for x then does not wait for the weight loads issued after it.
     constexpr int XP = xpre<NC>();
+    const int PIECE = 256 * mv_waves<TYPE, NC>();
     float4 xr[NC][XP];
 #pragma unroll
     for (int c = 0; c < NC; c++)
 #pragma unroll
-        for (int i = 0; i < XP; i++) xr[c][i] = load_x4(x + c * a.x_col_stride, 1024 * i + 4 * tid, K);
+        for (int i = 0; i < XP; i++) xr[c][i] = load_x4(x + c * a.x_col_stride, PIECE * i + 4 * tid, K);
     // the fused prologue's other operands come in with x: SwiGLU's second input and the norm weight
     float4 br[NC][XP], wr[XP];
     if (FUSED && a.glu_b) {
@@ -203,29 +267,30 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
 #pragma unroll
         for (int c = 0; c < NC; c++)
 #pragma unroll
-            for (int i = 0; i < XP; i++) br[c][i] = load_x4(gb + c * a.x_col_stride, 1024 * i + 4 * tid, K);
+            for (int i = 0; i < XP; i++) br[c][i] = load_x4(gb + c * a.x_col_stride, PIECE * i + 4 * tid, K);
     }
     if (FUSED && a.norm_w) {
 #pragma unroll
-        for (int i = 0; i < XP; i++) wr[i] = load_x4(a.norm_w, 1024 * i + 4 * tid, K);
+        for (int i = 0; i < XP; i++) wr[i] = load_x4(a.norm_w, PIECE * i + 4 * tid, K);
     }
 
     constexpr int G = 64 / LPR;  // rows in flight per wave
     const int lane = tid & 63, wave = tid >> 6;
     const int sub = lane % LPR, grp = lane / LPR;
-    const int64_t row = (int64_t)blockIdx.x * (4 * G) + wave * G + grp;
+    int64_t row = (int64_t)blockIdx.x * (NW * G) + wave * G + grp;
     const bool has_row = row < p.N;
     // Rows past the end load (and then ignore) the last row, chunks past the end the last chunk: the preloads carry no
     // lane-dependent branch, so they issue back to back.
-    const int64_t grow = p.row0 + (int64_t)mat * p.N + (has_row ? row : p.N - 1);
+    const int64_t row00 = p.row0 + (int64_t)mat * p.N;
+    int64_t grow = row00 + (has_row ? row : p.N - 1);
     const int nchunks = K / chunk_elems<TYPE>();
 
     // the residual the epilogue adds, requested now rather than after the reduction
-    const int64_t yoff = i12 * a.y_b2 + i13 * a.y_b3 + row;
+    const int64_t ybase = i12 * a.y_b2 + i13 * a.y_b3;
     float rr[NC];
     if (FUSED && p.res && has_row && sub == LPR - 1) {
 #pragma unroll
-        for (int c = 0; c < NC; c++) rr[c] = p.res[yoff + c * p.y_col_stride];
+        for (int c = 0; c < NC; c++) rr[c] = p.res[ybase + row + c * p.y_col_stride];
     }
 
     // weight chunks requested before the activation prologue, so the weight stream's first HBM round trip overlaps
@@ -246,62 +311,59 @@ __global__ __launch_bounds__(256) void k_matvec(MatvecArgs a) {
         if (a.glu_b || a.norm_w) {  // uniform: the fused prologue
             fused_prologue<TYPE, NC>(a, x, xi12, i13, xr, br, wr, xq, xd, xbs);
         } else {
-#pragma unroll
-            for (int c = 0; c < NC; c++) {
-                const float *xc = x + c * a.x_col_stride;
-#pragma unroll
-                for (int i = 0; i < XP; i++)
-                    if (1024 * i < K)
-                        quantize_piece<TYPE>(xr[c][i], 1024 * i, K, a.rounding, xq + c * K, xd + c * (K / XDB),
-                                             xbs + c * xbs_per_col<TYPE>(K));
-                for (int base = 1024 * XP; base < K; base += 1024)
-                    quantize_piece<TYPE>(load_x4(xc, base + 4 * tid, K), base, K, a.rounding, xq + c * K,
-                                         xd + c * (K / XDB), xbs + c * xbs_per_col<TYPE>(K));
-            }
+            plain_prologue<TYPE, NC>(a, x, xr, xq, xd, xbs);
         }
     } else {
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const float *xc = x + c * a.x_col_stride;
-#pragma unroll
-            for (int i = 0; i < XP; i++)
-                if (1024 * i < K) quantize_piece<TYPE>(xr[c][i], 1024 * i, K, a.rounding, xq + c * K, xd + c * (K / XDB),
-                                                       xbs + c * xbs_per_col<TYPE>(K));
-            for (int base = 1024 * XP; base < K; base += 1024)
-                quantize_piece<TYPE>(load_x4(xc, base + 4 * tid, K), base, K, a.rounding, xq + c * K,
-                                     xd + c * (K / XDB), xbs + c * xbs_per_col<TYPE>(K));
-        }
+        plain_prologue<TYPE, NC>(a, x, xr, xq, xd, xbs);
     }
     __syncthreads();
     if (!has_row) return;  // whole LPR-lane groups leave together; no barrier follows
 
-    float acc[NC];
+    while (true) {
+        float acc[NC];
 #pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = 0.0f;
+        for (int c = 0; c < NC; c++) acc[c] = 0.0f;
 #pragma unroll
-    for (int i = 0; i < PRE; i++) {
-        const int c = sub + i * LPR;
-        if (c < nchunks) dot_chunk<TYPE, NC, false>(pre[i], K, c, xq, xd, xbs, NC, acc);
-    }
-    if constexpr (TYPE == MX_TYPE_Q4_K) {  // a unit's registers are four chunks': one at a time
+        for (int i = 0; i < PRE; i++) {
+            const int c = sub + i * LPR;
+            if (c < nchunks) dot_chunk<TYPE, NC, false>(pre[i], K, c, xq, xd, xbs, NC, acc);
+        }
+        if constexpr (TYPE == MX_TYPE_Q4_K) {  // a unit's registers are four chunks': one at a time
 #pragma unroll 1
-        for (int c = sub + PRE * LPR; c < nchunks; c += LPR)
-            chunk_dot<TYPE, NC, false>(p.w, grow, K, c, xq, xd, xbs, NC, acc);
-    } else {
-#pragma unroll 4
-        for (int c = sub + PRE * LPR; c < nchunks; c += LPR)
-            chunk_dot<TYPE, NC, false>(p.w, grow, K, c, xq, xd, xbs, NC, acc);
-    }
-#pragma unroll
-    for (int c = 0; c < NC; c++) acc[c] = sum_lanes<LPR>(acc[c]);
-    if (sub == LPR - 1) {  // the lane holding the group's sum
-        float *y = p.y + yoff;
-        if (FUSED && p.res) {  // the residual ADD that follows the product, fused
-#pragma unroll
-            for (int c = 0; c < NC; c++) y[c * p.y_col_stride] = rr[c] + acc[c];
+            for (int c = sub + PRE * LPR; c < nchunks; c += LPR)
+                chunk_dot<TYPE, NC, false>(p.w, grow, K, c, xq, xd, xbs, NC, acc);
         } else {
+#pragma unroll 4
+            for (int c = sub + PRE * LPR; c < nchunks; c += LPR)
+                chunk_dot<TYPE, NC, false>(p.w, grow, K, c, xq, xd, xbs, NC, acc);
+        }
+        const int64_t next = row + (int64_t)gridDim.x * (NW * G);
+        const bool more = mv_loops<NC>() && next < p.N;
+        if (more) {  // the next rows' first chunks, ahead of this row's reduction and store
+            grow = row00 + next;
 #pragma unroll
-            for (int c = 0; c < NC; c++) y[c * p.y_col_stride] = acc[c];
+            for (int i = 0; i < PRE; i++) {
+                const int c = sub + i * LPR;
+                pre[i] = load_chunk<TYPE>(p.w, grow, K, c < nchunks ? c : nchunks - 1);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NC; c++) acc[c] = sum_lanes<LPR>(acc[c]);
+        if (sub == LPR - 1) {  // the lane holding the group's sum
+            float *y = p.y + ybase + row;
+            if (FUSED && p.res) {  // the residual ADD that follows the product, fused
+#pragma unroll
+                for (int c = 0; c < NC; c++) y[c * p.y_col_stride] = rr[c] + acc[c];
+            } else {
+#pragma unroll
+                for (int c = 0; c < NC; c++) y[c * p.y_col_stride] = acc[c];
+            }
+        }
+        if (!more) return;
+        row = next;
+        if (FUSED && p.res && sub == LPR - 1) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) rr[c] = p.res[ybase + row + c * p.y_col_stride];
         }
     }
 }
@@ -317,23 +379,48 @@ static int pick_lpr(int64_t nchunks, int preload, int forced) {
 }
 
 template <int TYPE, int NC, int LPR>
-static hipError_t launch_one(const MatvecArgs &a, int64_t maxN, size_t lds, hipStream_t s) {
+static hipError_t launch_one(const MatvecArgs &a, int64_t maxN, int nt, size_t lds, hipStream_t s) {
     constexpr int G = 64 / LPR;
-    dim3 grid((unsigned)((maxN + 4 * G - 1) / (4 * G)), (unsigned)a.nprob, (unsigned)a.nbatch);
+    const int R = nt / 64 * G;  // rows of a workgroup
     bool fused = a.glu_b || a.norm_w;
     for (int i = 0; i < a.nprob; i++) fused = fused || a.prob[i].res;
-    if (fused) hipLaunchKernelGGL((k_matvec<TYPE, NC, LPR, true>), grid, dim3(256), lds, s, a);
-    else hipLaunchKernelGGL((k_matvec<TYPE, NC, LPR, false>), grid, dim3(256), lds, s, a);
+    int64_t groups = (maxN + R - 1) / R;
+    if (mv_loops<NC>()) {
+        // Workgroups that go on to further rows, once there are more than the chip holds at a time: a fused kernel's
+        // registers leave room for one eight-wave workgroup per CU, a plain one's for two. Q8_0, five columns: gate and
+        // up of 2 x 6144 rows, K = 2048, behind a norm, as 256 / 384 / 768 workgroups 11.2 / 16.8 / 19.3 us; 151,936
+        // rows of K = 1024 as 256 / 512 / 768 / 4748 37.1 / 31.6 / 34.2 / 44.2 us.
+        int64_t total = 0;
+        for (int i = 0; i < a.nprob; i++) total += (a.prob[i].N + R - 1) / R;
+        const int64_t cap = fused ? 256 : 512, per = (total * a.nbatch + cap - 1) / cap;
+        groups = (groups + per - 1) / per;
+    }
+    dim3 grid((unsigned)groups, (unsigned)a.nprob, (unsigned)a.nbatch);
+    if (fused) hipLaunchKernelGGL((k_matvec<TYPE, NC, LPR, true>), grid, dim3((unsigned)nt), lds, s, a);
+    else hipLaunchKernelGGL((k_matvec<TYPE, NC, LPR, false>), grid, dim3((unsigned)nt), lds, s, a);
     return hipGetLastError();
 }
 
 template <int TYPE, int NC>
 static hipError_t launch_nc(const MatvecArgs &a, int64_t maxN, size_t lds, hipStream_t s) {
     const int64_t nchunks = a.K / chunk_elems<TYPE>();
-    switch (pick_lpr(nchunks, preload_of<TYPE>(), a.lpr)) {
-        case 16: return launch_one<TYPE, NC, 16>(a, maxN, lds, s);
-        case 32: return launch_one<TYPE, NC, 32>(a, maxN, lds, s);
-        default: return launch_one<TYPE, NC, 64>(a, maxN, lds, s);
+    int lpr = pick_lpr(nchunks, preload_of<TYPE>(), a.lpr);
+    // Four waves for K-quants of at most 1024 elements a row: a wave quantizes whole super-blocks, so that only four of
+    // eight would (Q6_K, 2 x 1024 rows, two columns behind a norm 5.7 us against 6.2).
+    const int nt = !mv_fixed<TYPE, NC>() && a.K <= 1024 ? 256 : mv_threads<TYPE, NC>();
+    if (nt > 256 && a.lpr == 0) {  // eight waves: fewer rows each rather than CUs left idle, while every lane has a chunk
+        auto groups = [&](int l) {
+            const int64_t rows = nt / l;
+            int64_t n = 0;
+            for (int i = 0; i < a.nprob; i++) n += (a.prob[i].N + rows - 1) / rows;
+            return n * a.nbatch;
+        };
+        while (lpr < 64 && nchunks >= 2 * lpr && groups(lpr) < 128) lpr *= 2;
+    }
+    switch (lpr) {
+        case 16: return launch_one<TYPE, NC, 16>(a, maxN, nt, lds, s);
+        case 32: return launch_one<TYPE, NC, 32>(a, maxN, nt, lds, s);
+        default: return launch_one<TYPE, NC, 64>(a, maxN, nt, lds, s);
     }
 }
 

@@ -148,8 +148,45 @@ __device__ __forceinline__ void wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory");
 }
 
+// The low bytes of four ints.
 __device__ __forceinline__ int pack4(int a, int b, int c, int d) {
-    return (a & 0xFF) | ((b & 0xFF) << 8) | ((c & 0xFF) << 16) | ((int)((unsigned)d << 24));
+    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)b, (uint32_t)a, 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)d, (uint32_t)c, 0x0c0c0400u);
+    return (int)__builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
+// ------------------------------------------------------------------------------------------------------------------
+// Correctly rounded quotients for the quantizers, without the scaling steps of a general division (Markstein's corrected
+// quotient: q = a r, q + r (a - b q)), and without a branch to one: the code of a general division that is never
+// reached still costs a decode step 25 us in 680, its instructions being fetched in 140 short kernels. The divisor's
+// mantissa is divided by and the exponent put back, which is exact while the quotient is normal or overflows. Each was
+// compared with the IEEE division over every finite or infinite float of its range on this chip.
+// ------------------------------------------------------------------------------------------------------------------
+__device__ __forceinline__ bool mid_range(float v) {  // |v| in [2^-60, 2^60)
+    return (__float_as_uint(v) & 0x7FFFFFFFu) - (67u << 23) < (120u << 23);
+}
+__device__ __forceinline__ float div127(float a) {  // a / 127, a finite
+    const float r = 1.0f / 127.0f, q = a * r;
+    return fmaf(fmaf(-127.0f, q, a), r, q);
+}
+__device__ __forceinline__ float recip_mid(float d) {  // 1 / d, d in mid_range
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
+__device__ __forceinline__ float recip_to126(float d) {  // 1 / d, 0 < |d| <= 2^126
+    return __builtin_amdgcn_ldexpf(recip_mid(__builtin_amdgcn_frexp_mantf(d)), -__builtin_amdgcn_frexp_expf(d));
+}
+__device__ __forceinline__ float quot127(float d) {  // 127 / d, d finite and not 0
+    const float m = __builtin_amdgcn_frexp_mantf(d), r = recip_mid(m), q = 127.0f * r;
+    return __builtin_amdgcn_ldexpf(fmaf(fmaf(-m, q, 127.0f), r, q), -__builtin_amdgcn_frexp_expf(d));
+}
+__device__ __forceinline__ bool zero_or_inf(float v) { return __builtin_amdgcn_classf(v, 0x264); }
+// (int)roundf(x * y) for |x y| < 2^17: half away from zero by adding the largest float below a half before truncating
+// (checked over every such float); the product rounds first.
+__device__ __forceinline__ int round_product(float x, float y) {
+#pragma clang fp contract(off)
+    const float v = x * y;
+    return (int)(v + copysignf(0x1.fffffep-2f, v));
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -157,7 +194,7 @@ __device__ __forceinline__ int pack4(int a, int b, int c, int d) {
 // the eight holds elements 4j..4j+3).
 //   REF (ggml-quants.c quantize_row_q8_{0,1}_ref): d = amax/127, id = d ? 1/d : 0, q = roundf(x*id).
 //   X86 (ggml-cpu x86 quantize_row_q8_{0,1}):       d = amax/127, id = amax ? 127/amax : 0, q = rint(x*id).
-// The divisions are IEEE (HIP's default correctly rounded fp32 division), the products single roundings.
+// The divisions are correctly rounded (the corrected quotients above), the products single roundings.
 // Returns the four quants packed in an int; *d gets fp32 d (unrounded), *sum the block's quant sum (all 8 lanes).
 // ------------------------------------------------------------------------------------------------------------------
 __device__ __forceinline__ int quant32_lane(float4 v, int rounding, float *d_out, int *sum_out) {
@@ -165,20 +202,20 @@ __device__ __forceinline__ int quant32_lane(float4 v, int rounding, float *d_out
     a = fmaxf(a, dpp_f<dpp::XOR1>(0.0f, a));
     a = fmaxf(a, dpp_f<dpp::XOR2>(0.0f, a));
     a = fmaxf(a, dpp_f<dpp::HALF_MIRROR>(0.0f, a));  // every lane of the eight now holds the block's amax
-    const float d = a / 127.0f;
+    const float d = a == INFINITY ? a : div127(a);
     int q0, q1, q2, q3;
     if (rounding == MX_ROUND_X86) {
-        const float id = a != 0.0f ? 127.0f / a : 0.0f;
+        const float id = zero_or_inf(a) ? 0.0f : quot127(a);
         q0 = (int)rintf(v.x * id);
         q1 = (int)rintf(v.y * id);
         q2 = (int)rintf(v.z * id);
         q3 = (int)rintf(v.w * id);
     } else {
-        const float id = d != 0.0f ? 1.0f / d : 0.0f;
-        q0 = (int)roundf(v.x * id);
-        q1 = (int)roundf(v.y * id);
-        q2 = (int)roundf(v.z * id);
-        q3 = (int)roundf(v.w * id);
+        const float id = zero_or_inf(d) ? 0.0f : recip_to126(d);
+        q0 = round_product(v.x, id);
+        q1 = round_product(v.y, id);
+        q2 = round_product(v.z, id);
+        q3 = round_product(v.w, id);
     }
     int s = q0 + q1 + q2 + q3;
     s += dpp_i<dpp::XOR1>(0, s);
@@ -221,7 +258,7 @@ __device__ __forceinline__ int quant256_wave(float4 v, int lane, float *d_out, i
     const int c = ((m0 >> L) & 1) ? 0 : (((m1 >> L) & 1) ? 1 : (((m2 >> L) & 1) ? 2 : 3));
     const float mine = c == 0 ? v.x : (c == 1 ? v.y : (c == 2 ? v.z : v.w));
     const float maxv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), L));
-    const float iscale = -127.0f / maxv;
+    const float iscale = zero_or_inf(maxv) ? -127.0f * __builtin_amdgcn_rcpf(maxv) : -quot127(maxv);
     int q[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -231,7 +268,7 @@ __device__ __forceinline__ int quant256_wave(float4 v, int lane, float *d_out, i
     int s = q[0] + q[1] + q[2] + q[3];
     s += dpp_i<dpp::XOR1>(0, s);
     s += dpp_i<dpp::XOR2>(0, s);
-    *d_out = 1.0f / iscale;
+    *d_out = mid_range(iscale) ? recip_mid(iscale) : 1.0f / iscale;  // (1 / iscale may be subnormal; uniform)
     *bsum_out = s;
     return pack4(q[0], q[1], q[2], q[3]);
 }

@@ -1,0 +1,82 @@
+"""Products of 1 to 8 columns on quantized weights (the mat-vec: eight waves a workgroup and workgroups that go on to
+further rows from two columns on), and the quantizers' divisions, on MI355X against the oracle.
+
+The bound of a product: the kernels sum the oracle's exact block integers, K / 32 scaled terms in fp32 in another order
+(at most 192 here), so about sqrt(192) * 2^-24 = 8e-7 of a row's largest output; 2e-5 would still show a lost term. Behind
+a norm or a GLU an activation that differs in its last bit may round to the next quant: one in 127 * 32 of a block's sum
+of squares, at most a few blocks a row, 2e-4.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from helpers import rel_err
+
+pytestmark = pytest.mark.gpu
+
+NAMES = {O.TYPE_Q8_0: "q8_0", O.TYPE_Q4_K: "q4_K", O.TYPE_Q5_K: "q5_K", O.TYPE_Q6_K: "q6_K"}
+TYPES = pytest.mark.parametrize("t", list(NAMES), ids=lambda t: NAMES[t])
+
+
+def weights(t, N, K, seed):
+    return O.quantize_chunk(t, O.fill_normal(seed, N, K, 0.0, 0.05))
+
+
+# rows at and around a workgroup's (8 waves x 1, 2 or 4 row groups), at the launch cap (512 workgroups, 32 rows each at
+# 256 elements, and one row more; one pass and two), K at one super-block, the four-wave rule (1024) and past the
+# preloaded pieces (2048 elements each)
+@TYPES
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 7, 8])
+@pytest.mark.parametrize("N,K", [(1, 256), (7, 1024), (8, 1280), (9, 4352), (33, 768), (129, 2304), (16385, 256), (8193, 512)])
+def test_columns(mx, be, t, M, N, K):
+    w, x = weights(t, N, K, 11 + N + K), O.fill_normal(13 + M, M, K)
+    W, X, Y = be.tensor(t, (K, N), w), be.tensor(mx.F32, (K, M), x), be.tensor(mx.F32, (N, M))
+    be.mul_mat(W, X, Y)
+    be.sync()
+    assert rel_err(Y.numpy().reshape(M, N), O.mul_mat(t, w, x)) <= 2e-5
+
+
+@TYPES
+@pytest.mark.parametrize("M", [1, 2, 5, 8])
+@pytest.mark.parametrize("Ns,K", [((70, 9, 1), 1024), ((4100, 8300), 512), ((2048, 1024, 1024), 2304)])
+def test_group_behind_a_norm(mx, be, t, M, Ns, K):
+    """Narrower problems of a group end early; the norm's sum over four and eight waves; residuals in place."""
+    ws = [weights(t, n, K, 17 + i) for i, n in enumerate(Ns)]
+    x, nw = O.fill_normal(19 + M, M, K) * np.float32(3), O.fill_normal(23, 1, K, 1.0, 0.1)[0]
+    r = [O.fill_normal(29 + i, M, n) for i, n in enumerate(Ns)]
+    W = [be.tensor(t, (K, n), w) for n, w in zip(Ns, ws)]
+    R = [be.tensor(mx.F32, (n, M), v) for n, v in zip(Ns, r)]
+    be.mul_mat_fused(W, be.tensor(mx.F32, (K, M), x), R, norm_w=be.tensor(mx.F32, (K,), nw), eps=1e-6, residual=R)
+    be.sync()
+    h = O.binary("mul", O.rms_norm(x, 1e-6), nw)
+    for n, w, v, y in zip(Ns, ws, r, R):
+        assert rel_err(y.numpy().reshape(M, n) - v, O.mul_mat(t, w, h)) <= 2e-4
+
+
+@TYPES
+@pytest.mark.parametrize("M", [2, 6])
+def test_glu(mx, be, t, M):
+    K, N = 3072, 1030
+    w, g, u = weights(t, N, K, 31), O.fill_normal(37, M, K), O.fill_normal(41, M, K)
+    W, G, U, Y = be.tensor(t, (K, N), w), be.tensor(mx.F32, (K, M), g), be.tensor(mx.F32, (K, M), u), be.tensor(mx.F32, (N, M))
+    be.mul_mat_fused([W], G, [Y], glu_b=U)
+    be.sync()
+    assert rel_err(Y.numpy().reshape(M, N), O.mul_mat(t, w, O.swiglu(g, u))) <= 2e-4
+
+
+@pytest.mark.parametrize("qt", [O.TYPE_Q8_0, O.TYPE_Q8_1, O.TYPE_Q8_K])
+@pytest.mark.parametrize("rounding", [O.ROUND_REF, O.ROUND_X86])
+def test_quantizers_over_all_exponents(mx, be, qt, rounding):
+    """Bit for bit from the smallest block maxima whose reciprocal is finite to 2^127, one exponent a row."""
+    if qt == O.TYPE_Q8_K and rounding == O.ROUND_X86:
+        pytest.skip("Q8_K has a single rounding")
+    K, es = 512, np.arange(-117, 127)
+    base = O.fill_normal(43, len(es), K)
+    base /= np.abs(base).max(axis=1, keepdims=True) * np.float32(1.01)  # the largest below 1
+    x = np.ldexp(base, es[:, None] + 1).astype(np.float32)
+    assert np.all(np.isfinite(x))
+    out = be.quantize_act(qt, rounding, be.tensor(mx.F32, (K, len(es)), x), K, len(es))
+    be.sync()
+    got = out.get_bytes()[: O.row_size(qt, K) * len(es)].reshape(len(es), -1)
+    want = O.quantize_rows(qt, x, rounding)
+    assert np.array_equal(got, want), f"rows differing: {es[(got != want).any(axis=1)]}"
