@@ -28,16 +28,20 @@ typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
 constexpr int KS = 128;       // K per LDS stage
 // Per tile: ring stages, blocks whose MFMAs a wave has in flight at once, and the waves per SIMD its registers are
-// allocated for. 64 x 64: four stages (70 KB, two workgroups per CU), block kb + 1's MFMAs issued before block kb's
-// VALU. 64 x 128: two stages (52 KB) and one block at a time (162 VGPRs), so three workgroups share a CU; measured at
-// M = 512 on the ASR gate/up group (768 workgroups) 50.7 -> 46.7 us against three stages and two blocks (212 VGPRs,
-// two workgroups per CU), while the 64 x 64 tile measured slower that way (down, K = 6144: 37.3 -> 40.8 us).
+// allocated for. What bounds both tiles is the VALU's conversion and fma per element and block (63% of the cycles at
+// M = 512, gate and up of 2 x 6144 rows, K = 2048; the matrix cores 22%), so its other instructions are kept few: 32-bit
+// index arithmetic, LDS offsets as immediates, scales of the idle lanes read as zeros instead of selected.
+// 64 x 64: three stages (54 KB, three workgroups per CU), block kb + 1's MFMAs issued before block kb's VALU. Against
+// four stages, two workgroups and 64-bit indexes: q / k / v of K = 2048 at M = 512 22.5 -> 21.5 us, gate and up at M = 130
+// 27.2 -> 23.2, down (K = 6144, N = 2048) at M = 512 36.3 -> 32.6.
+// 64 x 128: two stages (52 KB) and one block at a time, so three workgroups share a CU: 43.1 us at M = 512 on gate and
+// up, where the 64 x 64 tile takes 45.1, reading each operand more often.
 template <int BM, int BN>
 struct I8Cfg {
     static constexpr bool WIDE = BM == 64 && BN == 128;
-    static constexpr int NS = BM == 64 && BN == 64 ? 4 : (WIDE ? 2 : 3);
+    static constexpr int NS = WIDE ? 2 : 3;
     static constexpr int PD = BM == 64 && BN == 64 ? 2 : 1;
-    static constexpr int WPE = WIDE ? 3 : 2;
+    static constexpr int WPE = BM == 128 ? 1 : 3, WMIN = BN == 64 ? 3 : 1;
 };
 
 // Activation rows -> int8 quants [M][K], fp16 block scales [M][K/32] (d rounded to fp16, as the Q8_0 the weights
@@ -106,17 +110,19 @@ __device__ __forceinline__ _Float16 as_half(uint16_t b) {
 template <int BM, int BN>
 struct I8Lds {
     static constexpr int NS = I8Cfg<BM, BN>::NS;
-    static constexpr int SA = BM * KS, SB = BN * KS, SDX = BM * 8, SDW = BN * 8;  // slot sizes (bytes)
-    static constexpr int A = 0, B = A + NS * SA, DX = B + NS * SB, DW = DX + NS * SDX, SIZE = DW + NS * SDW;
+    // a slot: A, B, the scales of the activation rows and of the weight rows, eight zero bytes (the scales of the lanes
+    // whose k of the scale product is not 0)
+    static constexpr int A = 0, B = BM * KS, DX = B + BN * KS, DW = DX + BM * 8, ZERO = DW + BN * 8, SLOT = ZERO + 16;
+    static constexpr int SIZE = NS * SLOT;
     // copies per stage and wave: 16-byte ones of 8 quant rows each; 4-byte ones of 32 scale rows each, shared by the
     // waves (a wave past the last scale copy repeats it: the same bytes to the same place)
     static constexpr int QA = BM / 32, QB = BN / 32, NDX = BM / 32, NSC = (BM + BN) / 32, QS = (NSC + 3) / 4;
     static constexpr int OPS = QA + QB + QS;
     static_assert(SIZE <= 80 * 1024 || (BM == 128 && BN == 128), "two workgroups per CU");
-    static_assert(NS >= 2, "a ring of two stages or more");
+    static_assert(NS >= 2 && NS <= 4, "a ring of two to four stages");
 };
 
-__device__ __forceinline__ int i8_swz(int r) { return (r >> 1) & 7; }
+__device__ __forceinline__ uint32_t i8_swz(uint32_t r) { return (r >> 1) & 7; }
 
 // One wave's copies of a stage: per-lane byte offsets fixed for the whole K loop (rows past M or N clamped to the
 // last row), a per-stage uniform offset (k0 bytes of quants, k0 / 16 bytes of scales per row).
@@ -127,7 +133,7 @@ struct I8Dma {
     v4u ra, rb, rs[L::QS];
     uint32_t la, lb;  // LDS offsets of this wave's first A and B copy in a slot
 
-    __device__ __forceinline__ void init(int wave, const GemmArgs &g, const GemmProblem &pb, int64_t m0, int64_t n0) {
+    __device__ __forceinline__ void init(int wave, const GemmArgs &g, const GemmProblem &pb, uint32_t m0, uint32_t n0) {
         const int lane = threadIdx.x & 63;
         const uint32_t K = (uint32_t)g.K, nblk = K / 32, M = (uint32_t)g.M, N = (uint32_t)pb.N;
         ra = buf_rsrc(g.xq, M * K);
@@ -135,13 +141,13 @@ struct I8Dma {
         const v4u rdx = buf_rsrc(g.xd, M * nblk * 2), rdw = buf_rsrc(pb.w.p1, N * nblk * 2);
 #pragma unroll
         for (int q = 0; q < L::QA; q++) {
-            const int r = 8 * (wave * L::QA + q) + (lane >> 3);
-            a[q] = (uint32_t)min<int64_t>(m0 + r, M - 1) * K + 16u * (uint32_t)((lane & 7) ^ i8_swz(r));
+            const uint32_t r = 8 * (wave * L::QA + q) + (lane >> 3);
+            a[q] = min(m0 + r, M - 1) * K + 16u * ((uint32_t)(lane & 7) ^ i8_swz(r));
         }
 #pragma unroll
         for (int q = 0; q < L::QB; q++) {
-            const int r = 8 * (wave * L::QB + q) + (lane >> 3);
-            b[q] = (uint32_t)min<int64_t>(n0 + r, N - 1) * K + 16u * (uint32_t)((lane & 7) ^ i8_swz(r));
+            const uint32_t r = 8 * (wave * L::QB + q) + (lane >> 3);
+            b[q] = min(n0 + r, N - 1) * K + 16u * ((uint32_t)(lane & 7) ^ i8_swz(r));
         }
         la = (uint32_t)(wave * L::QA) * 1024u;
         lb = (uint32_t)(wave * L::QB) * 1024u;
@@ -149,9 +155,9 @@ struct I8Dma {
         for (int u = 0; u < L::QS; u++) {
             const int j = min(wave * L::QS + u, L::NSC - 1);  // scale copy j: DX rows 32 j .., then DW rows
             const bool isx = j < L::NDX;
-            const int r = 32 * (isx ? j : j - L::NDX) + (lane >> 1);
-            const int64_t row = isx ? min<int64_t>(m0 + r, M - 1) : min<int64_t>(n0 + r, N - 1);
-            s[u] = (uint32_t)row * nblk * 2u + 4u * (uint32_t)(lane & 1);
+            const uint32_t r = 32 * (isx ? j : j - L::NDX) + (lane >> 1);
+            const uint32_t row = isx ? min(m0 + r, M - 1) : min(n0 + r, N - 1);
+            s[u] = row * nblk * 2u + 4u * (uint32_t)(lane & 1);
             rs[u] = isx ? rdx : rdw;
             ls[u] = isx ? (uint32_t)(L::DX + 256 * j) : (uint32_t)(L::DW + 256 * (j - L::NDX));
         }
@@ -159,23 +165,20 @@ struct I8Dma {
 
     // stage k0 into ring slot `slot` (lds: the ring's LDS address)
     __device__ __forceinline__ void issue(uint32_t lds, int slot, int k0) const {
-        const uint32_t sa = lds + L::A + slot * L::SA + la, sb = lds + L::B + slot * L::SB + lb;
+        lds += (uint32_t)(slot * L::SLOT);
 #pragma unroll
-        for (int q = 0; q < L::QA; q++) dma16_lds(ra, sa + 1024u * q, a[q], (uint32_t)k0);
+        for (int q = 0; q < L::QA; q++) dma16_lds(ra, lds + L::A + la + 1024u * q, a[q], (uint32_t)k0);
 #pragma unroll
-        for (int q = 0; q < L::QB; q++) dma16_lds(rb, sb + 1024u * q, b[q], (uint32_t)k0);
+        for (int q = 0; q < L::QB; q++) dma16_lds(rb, lds + L::B + lb + 1024u * q, b[q], (uint32_t)k0);
 #pragma unroll
-        for (int u = 0; u < L::QS; u++) {
-            const uint32_t sl = ls[u] < (uint32_t)L::DW ? (uint32_t)(slot * L::SDX) : (uint32_t)(slot * L::SDW);
-            dma4_lds(rs[u], lds + ls[u] + sl, s[u], (uint32_t)(k0 / 16));
-        }
+        for (int u = 0; u < L::QS; u++) dma4_lds(rs[u], lds + ls[u], s[u], (uint32_t)(k0 / 16));
     }
 };
 
 // 32 x 32 accumulator layout of the 32x32 MFMAs: lane l, register r holds (row 8*(r/4) + 4*(l/32) + r%4, col l%32).
 template <int BM, int BN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, I8Cfg<BM, BN>::WPE))) void k_gemm_q8_0_i8(
-    GemmArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(I8Cfg<BM, BN>::WMIN, I8Cfg<BM, BN>::WPE))) void
+k_gemm_q8_0_i8(GemmArgs a) {
     using L = I8Lds<BM, BN>;
     constexpr int WM = BM / 2, WN = BN / 2;   // wave tile
     constexpr int TM = WM / 32, TN = WN / 32; // MFMA tiles per wave
@@ -184,28 +187,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, I8Cfg<BM
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t MT = (a.M + BM - 1) / BM;
-    int64_t per = 0;  // tiles of one split
+    // 32-bit throughout: rows x columns of the operands and the grid stay below 2^31
+    const uint32_t M = (uint32_t)a.M, MT = (M + BM - 1) / BM;
+    uint32_t per = 0;  // tiles of one split
 #pragma unroll
     for (int i = 0; i < 4; i++)
-        if (i < a.nprob) per += (a.prob[i].N + BN - 1) / BN * MT;
-    int64_t t = blockIdx.x;
+        if (i < a.nprob) per += ((uint32_t)a.prob[i].N + BN - 1) / BN * MT;
+    uint32_t t = blockIdx.x;
     const int split = (int)(t / per);
     t -= split * per;
     int pi = 0;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const int64_t ti = (a.prob[i].N + BN - 1) / BN * MT;
+        const uint32_t ti = ((uint32_t)a.prob[i].N + BN - 1) / BN * MT;
         if (pi == i && i + 1 < a.nprob && t >= ti) {
             t -= ti;
             pi = i + 1;
         }
     }
     const GemmProblem pb = problem(a, pi);
-    const int64_t ntp = (pb.N + BN - 1) / BN;
-    const int64_t m0 = (t / ntp) * BM, n0 = (t % ntp) * BN;
+    const uint32_t N = (uint32_t)pb.N, ntp = (N + BN - 1) / BN;
+    const uint32_t m0 = (t / ntp) * BM, n0 = (t % ntp) * BN;
     const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
-    const int nst = (int)(a.K / KS), sper = (nst + a.nsplit - 1) / a.nsplit;
+    const int nst = (int)a.K / KS, sper = (nst + a.nsplit - 1) / a.nsplit;
     const int kb0 = split * sper * KS, nloc = min(nst - split * sper, sper);  // this split's stages (never none)
 
     I8Dma<BM, BN> dma;
@@ -214,6 +218,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, I8Cfg<BM
     for (int s = 0; s < L::NS - 1; s++)
         if (s < nloc) dma.issue(lds, s, kb0 + s * KS);
 
+    if (tid < L::NS) *(uint2 *)(smem + tid * L::SLOT + L::ZERO) = make_uint2(0, 0);
     float acc[TM][TN][16];
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -224,24 +229,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, I8Cfg<BM
 
     // this lane's fragment offsets in a slot: row wm + 32 i + fr (A) or wn + 32 j + fr (B), chunk 2 kb + fh
     const int fr = lane & 31, fh = lane >> 5;
-    uint32_t aoff[TM][4], boff[TN][4], dxo[TM], dwo[TN];
+    // (every tile of a wave starts at a multiple of 32 rows, so one swizzle serves them all)
+    uint32_t aoff[4], boff[4], dxo[TM], dwo[TN];
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++) {
+        const uint32_t o = fr * KS + 16 * ((2 * kb + fh) ^ i8_swz(fr));
+        aoff[kb] = L::A + wm * KS + o;
+        boff[kb] = L::B + wn * KS + o;
+    }
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-        const int r = wm + 32 * i + fr;
-#pragma unroll
-        for (int kb = 0; kb < 4; kb++) aoff[i][kb] = (uint32_t)(r * KS + 16 * ((2 * kb + fh) ^ i8_swz(r)));
-        dxo[i] = (uint32_t)(r * 8);
+        const uint32_t r = wm + 32 * i + fr;
+        dxo[i] = fh ? L::ZERO : L::DX + r * 8;
     }
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-        const int r = wn + 32 * j + fr;
-#pragma unroll
-        for (int kb = 0; kb < 4; kb++) boff[j][kb] = (uint32_t)(r * KS + 16 * ((2 * kb + fh) ^ i8_swz(r)));
-        dwo[j] = (uint32_t)(r * 8);
+        const uint32_t r = wn + 32 * j + fr;
+        dwo[j] = fh ? L::ZERO : L::DW + r * 8;
     }
     const _Float16 hz = (_Float16)0.0f;
 
-    for (int s = 0; s < nloc; s++) {
+    auto stage = [&](int s, int slot) __attribute__((always_inline)) {
         // this wave's copies of stage s have landed (those of the stages after it that were issued may not), then
         // every wave's, and every wave has read the slot the next copies overwrite. The barrier is the bare
         // instruction: __syncthreads' release fence would wait for the copies still in flight too.
@@ -250,28 +258,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, I8Cfg<BM
         else if (L::NS > 3 && rem == 1) wait_vm<L::OPS>();
         else wait_vm<0>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (s + L::NS - 1 < nloc) dma.issue(lds, (s + L::NS - 1) % L::NS, kb0 + (s + L::NS - 1) * KS);
-        const int slot = s % L::NS;
-        const uint8_t *sa = smem + L::A + slot * L::SA, *sb = smem + L::B + slot * L::SB;
-        const uint8_t *sdx = smem + L::DX + slot * L::SDX, *sdw = smem + L::DW + slot * L::SDW;
-        // every fragment and scale of the stage first, so the reads overlap each other and the MFMAs that follow
+        if (s + L::NS - 1 < nloc) dma.issue(lds, (slot + L::NS - 1) % L::NS, kb0 + (s + L::NS - 1) * KS);
+        const uint8_t *ring = smem + slot * L::SLOT;
+        constexpr int PD = I8Cfg<BM, BN>::PD;
+        // every fragment and scale of the stage first, so the reads overlap each other and the MFMAs that follow (with one
+        // block in flight the weight fragments of the last two blocks later: registers)
         v4i af[4][TM], bf[4][TN];
         uint2 dx4[TM], dw4[TN];  // the row's (column's) four fp16 block scales
 #pragma unroll
         for (int i = 0; i < TM; i++) {
-            dx4[i] = *(const uint2 *)(sdx + dxo[i]);
+            dx4[i] = *(const uint2 *)(ring + dxo[i]);
 #pragma unroll
-            for (int kb = 0; kb < 4; kb++) af[kb][i] = *(const v4i *)(sa + aoff[i][kb]);
+            for (int kb = 0; kb < 4; kb++) af[kb][i] = *(const v4i *)(ring + aoff[kb] + 32 * i * KS);
         }
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            dw4[j] = *(const uint2 *)(sdw + dwo[j]);
+            dw4[j] = *(const uint2 *)(ring + dwo[j]);
 #pragma unroll
-            for (int kb = 0; kb < 4; kb++) bf[kb][j] = *(const v4i *)(sb + boff[j][kb]);
+            for (int kb = 0; kb < (PD == 2 ? 4 : 2); kb++) bf[kb][j] = *(const v4i *)(ring + boff[kb] + 32 * j * KS);
         }
         // block kb's integer sums and scale products; with PD = 2 block kb + 1's MFMAs are issued before block kb's
         // conversions and fmas, so the matrix cores and the VALU overlap within the wave
-        constexpr int PD = I8Cfg<BM, BN>::PD;
         v16i S[PD][TM][TN];
         v16f C[PD][TM][TN];
         auto mfma = [&](int kb, int d) {
@@ -279,12 +286,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, I8Cfg<BM
 #pragma unroll
             for (int i = 0; i < TM; i++) {
                 const uint32_t w = kb < 2 ? dx4[i].x : dx4[i].y;
-                as[i] = v4h{fh ? hz : as_half((uint16_t)(kb & 1 ? w >> 16 : w & 0xFFFF)), hz, hz, hz};
+                as[i] = v4h{as_half((uint16_t)(kb & 1 ? w >> 16 : w & 0xFFFF)), hz, hz, hz};
             }
 #pragma unroll
             for (int j = 0; j < TN; j++) {
                 const uint32_t w = kb < 2 ? dw4[j].x : dw4[j].y;
-                bs[j] = v4h{fh ? hz : as_half((uint16_t)(kb & 1 ? w >> 16 : w & 0xFFFF)), hz, hz, hz};
+                bs[j] = v4h{as_half((uint16_t)(kb & 1 ? w >> 16 : w & 0xFFFF)), hz, hz, hz};
             }
             const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
             const v16f fz = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -307,10 +314,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, I8Cfg<BM
         mfma(0, 0);
 #pragma unroll
         for (int kb = 0; kb < KS / 32; kb++) {
+            if (PD == 1 && kb + 2 < KS / 32) {
+#pragma unroll
+                for (int j = 0; j < TN; j++) bf[kb + 2][j] = *(const v4i *)(ring + boff[kb + 2] + 32 * j * KS);
+            }
             if (PD == 2 && kb + 1 < KS / 32) mfma(kb + 1, (kb + 1) % PD);
             fold(kb % PD);
             if (PD == 1 && kb + 1 < KS / 32) mfma(kb + 1, 0);
         }
+    };
+    // stage s in slot s % NS. The 64 x 64 tile has the slots written out, so that their offsets are the LDS reads'
+    // immediates; the wider ones have no registers for what the compiler then moves from stage to stage (spills, 77 us
+    // instead of 43).
+    if constexpr (BM == 64 && BN == 64) {
+        for (int s = 0;;) {
+            stage(s, 0);
+            if (++s >= nloc) break;
+            stage(s, 1);
+            if (++s >= nloc) break;
+            stage(s, 2);
+            if (++s >= nloc) break;
+        }
+    } else {
+        for (int s = 0; s < nloc; s++) stage(s, s % L::NS);
     }
 
     float *y = pb.y;
@@ -320,17 +346,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, I8Cfg<BM
         ldy = a.ntot;
     }
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+    for (int i = 0; i < TM; i++) {
+        // row m = m0 + wm + 32 i + 4 (lane / 32) + 8 (r / 4) + r % 4: one pointer a lane, uniform steps
+        const uint32_t mr = m0 + wm + 32 * i + 4 * fh;
+        float *yr = y + (int64_t)mr * ldy + n0 + wn + fr;
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int64_t n = n0 + wn + 32 * j + fr;
-            if (n >= pb.N) continue;
+        for (int r = 0; r < 16; r++) {
+            const uint32_t dm = 8 * (r >> 2) + (r & 3);
+            if (mr + dm >= M) continue;
+            float *p = yr + dm * ldy;
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int64_t m = m0 + wm + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (m < a.M) y[m * ldy + n] = acc[i][j][r];
-            }
+            for (int j = 0; j < TN; j++)
+                if (n0 + wn + 32 * j + fr < N) p[32 * j] = acc[i][j][r];
         }
+    }
 }
 
 // y[m][col] = the nsplit partials of (m, col) added in split order (split 0 first); one thread per column.
