@@ -47,7 +47,7 @@ struct FmLds {
     static constexpr int STAT = FM_W * FM_P * 8, OUT = STAT + FM_W * FM_P * OS * 4;
     static constexpr int Q = RING, END = Q + FM_P * RB;  // the pairs' q rows in fp16, laid out as a key tile
     static constexpr int SIZE = END > OUT ? END : OUT;
-    static_assert(SIZE <= 160 * 1024, "LDS");
+    static_assert(SIZE <= 160 * 1024 && OUT + FM_W * (D + 64) * 4 <= SIZE, "LDS");
 };
 
 // Chunk c of K row r lies at c ^ fm_swk(r), of V row r at c ^ fm_swv(r): the rows of a key fragment read (16 at one
@@ -83,6 +83,74 @@ __device__ __forceinline__ float fm_rest1(v2h h, float p) {
     float d;
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(h), "v"(p));
     return d;
+}
+
+// One wave's sums of head h, row i over a split's positions, in fp32 and over the positions that the row sees alone
+// (qs [D], ps [64]: LDS of its own). k_fa_mfma's second form where values are infinities or NaN, so small rather than fast.
+template <int D>
+__device__ __forceinline__ void fa_row_alone(const FaArgs &a, int64_t split, int64_t h, int64_t i, int lane, float *qs,
+                                             float *ps) {
+    constexpr int DL = D / 64, NV = 16;  // channels per lane; value rows in flight
+    auto own = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+    const int64_t hk = h / a.gqa, j0 = split * a.split_len, j1 = min(a.n_kv, j0 + a.split_len);
+    const uint8_t *kb = (const uint8_t *)a.k + hk * a.k_nb2, *vb = (const uint8_t *)a.v + hk * a.v_nb2;
+    const uint16_t *mrow = a.mask ? (const uint16_t *)((const uint8_t *)a.mask + i * a.m_nb1) : nullptr;
+    const float *q = (const float *)((const uint8_t *)a.q + i * a.q_nb1 + h * a.q_nb2);
+    own();
+#pragma unroll
+    for (int c = 0; c < DL; c++) qs[64 * c + lane] = h2f(f2h(q[64 * c + lane]));
+    own();
+    float M = -INFINITY, S = 0.0f, acc[DL] = {};
+    for (int64_t base = j0; base < j1; base += 64) {
+        const int64_t j = base + lane;
+        const float m = j < j1 ? (mrow ? h2f(mrow[j]) : 0.0f) : -INFINITY;
+        float s = -INFINITY;
+        if (m != -INFINITY) {
+            const v8h *kr = (const v8h *)(kb + j * a.k_nb1);
+            float dot = 0.0f;
+#pragma unroll 4
+            for (int c = 0; c < D / 8; c++) {
+                const v8h w = kr[c];
+#pragma unroll
+                for (int e = 0; e < 8; e++) dot = fmaf((float)w[e], qs[8 * c + e], dot);
+            }
+            s = dot * a.scale + m;
+        }
+        const float mc = wave_max_f(s);
+        if (mc == -INFINITY && !__any(s != s)) continue;  // uniform: nothing of the chunk is seen
+        const float Mn = fmaxf(M, mc), r = M == Mn ? 1.0f : expf(M - Mn), p = expf(s - Mn);
+        S = S * r + wave_sum_f(s == -INFINITY ? 0.0f : p);
+        M = Mn;
+        own();
+        ps[lane] = s == -INFINITY ? -1.0f : p;
+        own();
+#pragma unroll
+        for (int c = 0; c < DL; c++) acc[c] *= r;
+#pragma unroll 1
+        for (int t0 = 0; t0 < 64; t0 += NV) {
+            _Float16 v[NV][DL];
+#pragma unroll
+            for (int t = 0; t < NV; t++)
+#pragma unroll
+                for (int c = 0; c < DL; c++)
+                    v[t][c] = ((const _Float16 *)(vb + min(base + t0 + t, j1 - 1) * a.v_nb1))[64 * c + lane];
+#pragma unroll
+            for (int t = 0; t < NV; t++) {
+                const float pt = ps[t0 + t];
+#pragma unroll
+                for (int c = 0; c < DL; c++) acc[c] = pt < 0.0f ? acc[c] : fmaf(pt, (float)v[t][c], acc[c]);
+            }
+        }
+    }
+    const float inv = a.nsplit > 1 ? 1.0f : (S == 0.0f ? 0.0f : 1.0f / S);
+    float *part = a.part + ((i * a.n_head + h) * a.nsplit + split) * (D + 2);
+    float *o = a.nsplit > 1 ? part + 2 : a.dst + (i * a.n_head + h) * D;
+#pragma unroll
+    for (int c = 0; c < DL; c++) o[64 * c + lane] = acc[c] * inv;
+    if (a.nsplit > 1 && lane == 0) {
+        part[0] = M;
+        part[1] = S;
+    }
 }
 
 template <int D, bool MASK>
@@ -328,6 +396,7 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
     __syncthreads();
     constexpr int TP = 64 * FM_W / (D / 4);  // pairs in a round of the threads, four channels each
     const int d4 = 4 * (tid % (D / 4));
+    bool odd = false;  // a sum that is not finite
 #pragma unroll
     for (int pr = tid / (D / 4); pr < FM_P; pr += TP) {
         const uint32_t p = p0 + (uint32_t)pr, i = p / gqa;
@@ -340,6 +409,8 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
             Ls += st_l[w * FM_P + pr];
             x += *(const v4f *)(os + (w * FM_P + pr) * L::OS + d4);
         }
+#pragma unroll
+        for (int c = 0; c < 4; c++) odd |= !(fabsf(x[c]) < INFINITY);
         const int64_t row = i * a.n_head + hk * a.gqa + (p - i * gqa);
         if (a.nsplit == 1) {
             const float inv = Ls == 0.0f ? 0.0f : 1.0f / Ls;
@@ -353,6 +424,18 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
                 part[1] = Ls;
             }
         }
+    }
+    // An infinity or a NaN among the values reaches pairs that do not see its position (0 times it is NaN), and as NaN
+    // those that see an infinity (times the halves of its weight). Then this wave forms its pairs' sums again, one by one
+    // over the positions that each sees.
+    if (!__any(odd)) return;
+    wait_vm<0>();  // the stores above come first
+    constexpr int PW = 64 / (D / 4);  // pairs of a wave in a round
+    float *qs = (float *)(smem + L::OUT) + wave * (D + 64);
+#pragma unroll 1
+    for (int e = 0; e < FM_P / FM_W; e++) {
+        const uint32_t p = p0 + (uint32_t)(e / PW * TP + wave * PW + e % PW), i = p / gqa;
+        if (p < np) fa_row_alone<D>(a, split, hk * a.gqa + (p - i * gqa), i, lane, qs, qs + D);
     }
 }
 

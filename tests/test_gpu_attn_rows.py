@@ -129,6 +129,30 @@ def test_not_a_number(mx, be):
     assert np.isnan(got[5, 1]).all() and np.isfinite(np.delete(got, 5, 0)).all() and np.isfinite(got[5, 0]).all()
 
 
+@pytest.mark.parametrize("heads,kv,D", [(2, 1, 128), (16, 8, 128), (6, 2, 128), (4, 2, 64), (3, 3, 64)])
+@pytest.mark.parametrize("odd", ["nan", "inf", "-inf", "both", "key"])
+def test_hidden_odd_values(mx, be, heads, kv, D, odd):
+    """Infinities and NaN reach the rows that see their position and no other: positions that some rows of a workgroup see
+    (causal; 77 hidden from the first rows), and one that no row sees in a step with positions that some do."""
+    rows, n_kv, past = 70, 400, 220
+    q, k, v, mask = case(rows, n_kv, heads, kv, D, 5, past)
+    mask[:9, 77] = -np.inf
+    want, bound = exact(q, k, v, mask, D ** -0.5)
+    at = [77, past + 3, past + 40, past + rows + 5]
+    for i, j in enumerate(at):
+        (k if odd == "key" else v)[j, :, ::3] = np.nan if odd == "key" else (np.inf, -np.inf)[i % 2] if odd == "both" else float(odd)
+    for i in range(rows):  # what the odd values that a row sees add to the sums of its others
+        for j in at:
+            if mask[i, j] == 0:
+                with np.errstate(invalid="ignore"):
+                    want[i] += np.nan if odd == "key" else np.where(np.isfinite(v[j]), 0, v[j]).repeat(heads // kv, 0)
+    got = device(mx, be, q, k, v, mask, D ** -0.5, cap=n_kv + 8)
+    inf = np.isinf(want)  # (NaN where the merge of splits multiplies it by a split's weight of 0)
+    assert np.isnan(got[np.isnan(want)]).all() and np.all(np.isnan(got[inf]) | (got[inf] == want[inf]))
+    ok = np.isfinite(want)  # (channels without odd values are whole in every row)
+    assert ok[:3].all() and np.all(np.abs(got[ok] - want[ok]) <= np.broadcast_to(bound, want.shape)[ok])
+
+
 def test_recorded(mx):
     """Recorded with no eager run before it (splits need scratch: the row kernel takes it), then after one; replayed."""
     be = mx.Backend(0)
