@@ -9,14 +9,16 @@
 //
 // Per step: S^T = K Q^T (v_mfma_f32_32x32x16_f16; a lane ends up with 16 positions of one pair, so the row maximum and
 // sum are register reductions and one exchange), softmax in fp32, O^T += V^T P^T with V read transposed from LDS
-// (ds_read_b64_tr_b16). The probabilities stay fp32: each is multiplied in as the sum of two fp16 values, hi + lo,
-// scaled by about 2^7 so that lo keeps full precision (22 bits and a sign together, as near as fp32's 24 bits round).
-// The running maximum is a reference that moves only when a score passes it by a factor of 2^8 (p then stays below
-// 2^15 in fp16), so the accumulators are rarely rescaled.
+// (ds_read_b64_tr_b16). A weight is multiplied in as the sum of two fp16 values, hi + lo, scaled by 2^13 so that lo keeps
+// full precision: 23 bits together, where the weight itself, an exponential rounded to 24, is good to about as many.
+// The running maximum is a reference that moves only when a score passes it by more than 2 (weights then stay below e^2,
+// 2^16 in fp16), so the accumulators are rarely rescaled; a larger margin would cost the large weights' exponents bits.
+// Error against double precision over 64 shapes of 2 to 512 rows, relative to the one-row kernels': 0.50 of it on
+// (geometric) average; with exact scores, few positions: 7.3e-8 against 7.7e-8.
 //
 // What bounds it: the VALU, at about 14 issue slots a score against 6 of the matrix cores (two waves per SIMD). 512 rows
-// at 1024 positions before them, 16 heads on 8 of 128: 376 us with one workgroup per row (k_fa_gqa), 16-21 us here (four
-// waves and a two-slot ring 29.6; q not staged through LDS and the rescale inside the loop 25.5).
+// at 1024 positions before them, 16 heads on 8 of 128: 19.4 us (four waves and a two-slot ring 29.6; q not staged through LDS and the rescale
+// inside the loop 25.5); one workgroup per row (k_fa_gqa), with the q / k norms, RoPE and stores before it, 365.
 #include "mx_common.h"
 #include "mx_device.h"
 
@@ -73,16 +75,11 @@ __device__ __forceinline__ float half_sum(float v) {
     return __uint_as_float(a) + __uint_as_float(b);
 }
 
-// p minus the low / high half of h, in one instruction (left to the compiler: a conversion and a subtraction)
-__device__ __forceinline__ float fm_rest0(v2h h, float p) {
-    float d;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(d) : "v"(h), "v"(p));
-    return d;
-}
-__device__ __forceinline__ float fm_rest1(v2h h, float p) {
-    float d;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(h), "v"(p));
-    return d;
+// fp16 of a times s and of b times s, in two instructions (left to the compiler: two products and a conversion)
+__device__ __forceinline__ v2h fm_halves(float a, float b, float s) {
+    v2h h;
+    asm("v_fma_mixlo_f16 %0, %1, %3, 0\n\tv_fma_mixhi_f16 %0, %2, %3, 0" : "=&v"(h) : "v"(a), "v"(b), "s"(s));
+    return h;
 }
 
 // One wave's sums of head h, row i over a split's positions, in fp32 and over the positions that the row sees alone
@@ -247,7 +244,7 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
     for (int dt = 0; dt < DT; dt++) O[dt] = zero;
     float Mr = -INFINITY, l = 0.0f;  // the reference exponent and this lane's half of the row's sum
     constexpr float LOG2E = 1.44269504f, LN2 = 0.693147181f;
-    constexpr float REF = 4.8520303f, PASS = 10.3972077f;  // 7 ln 2, 15 ln 2
+    constexpr float PSCALE = 0x1p13f;  // of the weights on their way to fp16: at most e^2, so below fp16's largest
 
     const uint8_t *sl = smem + wave * L::SLOT;
     v16f S;                 // register r of lane l: position 8 (r / 4) + 4 fh + r % 4 of the step, pair fr
@@ -311,8 +308,8 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
                 }
                 plain = !__any(ml == -INFINITY);
                 mc = half_max(mc) * sc;
-                const bool need = mc > Mr + PASS;  // (always from Mr = -inf, once a score is finite)
-                Mn = need ? mc - REF : Mr;
+                const bool need = mc > Mr + 2.0f;  // (always from Mr = -inf, once a score is finite)
+                Mn = need ? mc : Mr;
                 formed = true;
                 if (__any(need)) {
                     rescale = true;
@@ -339,12 +336,11 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
             v8h hi[2], lo[2];
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
-                const v2h h = __builtin_convertvector((v2f{p[r], p[r + 1]}), v2h);
-                const v2h d = __builtin_convertvector((v2f{fm_rest0(h, p[r]), fm_rest1(h, p[r + 1])}), v2h);
+                const v2h h = fm_halves(p[r], p[r + 1], PSCALE);
                 hi[r >> 3][r & 7] = h[0];
                 hi[r >> 3][(r & 7) + 1] = h[1];
-                lo[r >> 3][r & 7] = d[0];
-                lo[r >> 3][(r & 7) + 1] = d[1];
+                lo[r >> 3][r & 7] = (_Float16)fmaf(p[r], PSCALE, -(float)h[0]);
+                lo[r >> 3][(r & 7) + 1] = (_Float16)fmaf(p[r + 1], PSCALE, -(float)h[1]);
             }
             if (more) wait_vm<OPS_K>();  // the values have landed (the next keys, issued after them, may not)
             else wait_vm<0>();
@@ -390,7 +386,7 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
         for (int u = 0; u < 4; u++) {  // channels 32 dt + 8 u + 4 fh .. + 3
             v4f x;
 #pragma unroll
-            for (int c = 0; c < 4; c++) x[c] = O[dt][4 * u + c] * f;
+            for (int c = 0; c < 4; c++) x[c] = O[dt][4 * u + c] * (f * (1.0f / PSCALE));
             *(v4f *)(os + (wave * FM_P + fr) * L::OS + 32 * dt + 8 * u + 4 * fh) = x;
         }
     __syncthreads();

@@ -153,6 +153,23 @@ def test_hidden_odd_values(mx, be, heads, kv, D, odd):
     assert ok[:3].all() and np.all(np.abs(got[ok] - want[ok]) <= np.broadcast_to(bound, want.shape)[ok])
 
 
+@pytest.mark.parametrize("heads,kv,D", [(8, 1, 128), (12, 4, 128), (8, 1, 64), (16, 16, 64)])
+def test_weights_in_full(mx, be, heads, kv, D):
+    """Scores that are exact in fp32 (one product each), so that the error is the weights' own and that of their sums. A
+    weight is off by half a unit of its exponent where that is below 2 (2^-24), of its exponential (2^-24) and of its two
+    fp16 parts (2^-24 of most of them), the sum, the division and the product by 2^-25 each: root mean square about
+    1.2 * 2^-24 = 7.3e-8 of a result of one to some ten weights. Exponents of 4 to 8 (units of 2^-21) would add 1.2e-7."""
+    g = np.random.default_rng(D)
+    rows = 72
+    q, k, v, mask = case(rows, rows, heads, kv, D, 1, 0)
+    q[:] = 0
+    np.put_along_axis(q, g.integers(0, D, (rows, heads, 1)), 8 * g.uniform(1, 2, (rows, heads, 1)).astype(np.float16), 2)
+    k = g.uniform(-0.5, 0.5, k.shape).astype(np.float16)
+    want, _ = exact(q, k, v, mask, 0.125)
+    got = device(mx, be, q, k, v, mask, 0.125)
+    assert np.square(got[:48] - want[:48]).sum() <= (1e-7) ** 2 * np.square(want[:48]).sum()
+
+
 def test_recorded(mx):
     """Recorded with no eager run before it (splits need scratch: the row kernel takes it), then after one; replayed."""
     be = mx.Backend(0)
