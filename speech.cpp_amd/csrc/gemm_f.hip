@@ -30,9 +30,10 @@ struct FgProblem {
     float *y;
     int64_t ldy;  // floats between consecutive m rows of y
 };
-// Up to four weights sharing the activations. The grid is one dimension: split after split, problem after problem, the
-// problem's tiles with n fastest. Split s covers the stages [s per, (s + 1) per) and, with nsplit > 1, writes partial
-// sums to ws ([nsplit][M][ntot], problem p from column col0[p]), which k_fg_reduce adds in split order.
+// Up to four weights sharing the activations, or one weight (prob[0]) over batch slices. A slice's tiles are the grid's
+// first dimension: split after split, problem after problem, the problem's tiles with n fastest; the slices are its second
+// (the pass's and the reduce's third). Split s covers the stages [s per, (s + 1) per) and, with nsplit > 1, writes partial
+// sums to ws ([slice][nsplit][M][ntot], problem p from column col0[p]), which k_fg_reduce adds in split order.
 struct FgArgs {
     FgProblem prob[4];
     int nprob, nsplit;
@@ -41,15 +42,33 @@ struct FgArgs {
     int64_t x_nb;  // bytes between activation rows
     int64_t ntot, col0[4];
     float *ws;
+    int batched;      // several slices (what follows is read only then)
+    uint32_t z0, ne2, r2, r3;  // the launch's first slice; slices along axis 2, and to a matrix of the weight
+    int64_t x_b2, x_b3, w_b2, w_b3, y_b2, y_b3;  // bytes between slices (the fp16 rows: x_b2, the launch's one after another)
 };
 
+// A launch's slice `rel` along the batch axes.
+struct FgSlice {
+    uint32_t i2, i3;
+};
+__device__ __forceinline__ uint32_t fg_uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ FgSlice fg_slice(const FgArgs &a, uint32_t rel) {
+    const uint32_t z = a.z0 + rel, i3 = z / a.ne2;
+    return FgSlice{fg_uniform(z - i3 * a.ne2), fg_uniform(i3)};
+}
+
 // x rows (f32) -> fp16 rows [M][K], round to nearest even, as ggml_cpu_fp32_to_fp16 makes src1 of F16 weights.
-__global__ __launch_bounds__(256) void k_f16_act(const float *x, int64_t x_stride, int64_t K, uint16_t *xh) {
+__global__ __launch_bounds__(256) void k_f16_act(const float *x, int64_t x_stride, int64_t K, uint16_t *xh, FgArgs a) {
+    if (a.batched) {
+        const FgSlice z = fg_slice(a, blockIdx.z);
+        x = (const float *)((const uint8_t *)x + z.i2 * a.x_b2 + z.i3 * a.x_b3);
+        xh += (int64_t)blockIdx.z * a.M * K;
+    }
     const int64_t m = blockIdx.x, e = ((int64_t)blockIdx.y * 256 + threadIdx.x) * 8;
     if (e >= K) return;
-    const float4 a = *(const float4 *)(x + m * x_stride + e), b = *(const float4 *)(x + m * x_stride + e + 4);
-    v8h h = {(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w,
-             (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
+    const float4 u = *(const float4 *)(x + m * x_stride + e), v = *(const float4 *)(x + m * x_stride + e + 4);
+    v8h h = {(_Float16)u.x, (_Float16)u.y, (_Float16)u.z, (_Float16)u.w,
+             (_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
     *(v8h *)(xh + m * K + e) = h;
 }
 
@@ -81,7 +100,7 @@ struct FgCfg {
     static constexpr int CA = SA / 1024, CB = SB / 1024, OPS = KG * (CA + CB) / NW;
     // Sums of sums: see the kernel. Three levels where the accumulators are few.
     static constexpr bool MID = TM * TN * NR <= 32;
-    static_assert(KG * (CA + CB) % NW == 0 && WM % T == 0 && WN % T == 0, "tile");
+    static_assert(NW <= 8 && KG * (CA + CB) % NW == 0 && WM % T == 0 && WN % T == 0, "tile");
     static_assert(LDS <= 160 * 1024 && NS >= 2, "LDS");
     static_assert((KG - 1) * WGM * WGN * TM * TN * NR * 256 <= LDS, "the groups' sums fit the ring");
 };
@@ -109,8 +128,14 @@ __global__ __launch_bounds__(64 * C::NW) void k_gemm_f(FgArgs a) {
             pi = i + 1;
         }
     }
-    const uint8_t *w = fg_pick(pi, a.prob[0].w, a.prob[1].w, a.prob[2].w, a.prob[3].w);
+    const uint8_t *w = fg_pick(pi, a.prob[0].w, a.prob[1].w, a.prob[2].w, a.prob[3].w), *x = a.x;
     const int64_t N = fg_pick(pi, a.prob[0].N, a.prob[1].N, a.prob[2].N, a.prob[3].N);
+    FgSlice z = {0, 0};
+    if (a.batched) {
+        z = fg_slice(a, blockIdx.y);
+        w += fg_uniform(z.i2 / a.r2) * a.w_b2 + fg_uniform(z.i3 / a.r3) * a.w_b3;
+        x += C::H && !C::XF ? blockIdx.y * a.x_b2 : z.i2 * a.x_b2 + z.i3 * a.x_b3;
+    }
     const int64_t ntp = (N + C::BN - 1) / C::BN;
     // (the divisions run on the vector unit: their uniform results go back to scalar registers for the copies' operands)
     const int mt = __builtin_amdgcn_readfirstlane((int)(t / ntp)), nt = __builtin_amdgcn_readfirstlane((int)(t % ntp));
@@ -123,7 +148,7 @@ __global__ __launch_bounds__(64 * C::NW) void k_gemm_f(FgArgs a) {
     // This wave's copies of a stage: copy q = wave OPS + j of the stage's KG x (CA + CB), each slice's activations first;
     // a weight copy is 8 rows of 128 bytes, an activation copy 8 rows of 128 or 4 of 256 bytes.
     const int64_t row_b = a.K * C::ES, row_a = C::XF || !C::H ? a.K * 4 : a.K * 2;
-    const v4u ra = buf_rsrc(a.x + m0 * a.x_nb, (uint32_t)((min<int64_t>(C::BM, a.M - m0) - 1) * a.x_nb + row_a));
+    const v4u ra = buf_rsrc(x + m0 * a.x_nb, (uint32_t)((min<int64_t>(C::BM, a.M - m0) - 1) * a.x_nb + row_a));
     const v4u rb = buf_rsrc(w + n0 * row_b, (uint32_t)(min<int64_t>(C::BN, N - n0) * row_b));
     uint32_t voff[C::OPS];
 #pragma unroll
@@ -324,8 +349,10 @@ __global__ __launch_bounds__(64 * C::NW) void k_gemm_f(FgArgs a) {
     float *y = fg_pick(pi, a.prob[0].y, a.prob[1].y, a.prob[2].y, a.prob[3].y);
     int64_t ldy = fg_pick(pi, a.prob[0].ldy, a.prob[1].ldy, a.prob[2].ldy, a.prob[3].ldy);
     if (a.nsplit > 1) {  // this split's partial sums
-        y = a.ws + (int64_t)split * a.M * a.ntot + fg_pick(pi, a.col0[0], a.col0[1], a.col0[2], a.col0[3]);
+        y = a.ws + ((int64_t)blockIdx.y * a.nsplit + split) * a.M * a.ntot + fg_pick(pi, a.col0[0], a.col0[1], a.col0[2], a.col0[3]);
         ldy = a.ntot;
+    } else if (a.batched) {
+        y = (float *)((uint8_t *)y + z.i2 * a.y_b2 + z.i3 * a.y_b3);
     }
     // accumulators: 32 x 32 lane l, register r: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32; 16 x 16: row
     // 4 (l / 16) + r, column l % 16
@@ -348,13 +375,17 @@ __global__ __launch_bounds__(256) void k_fg_reduce(FgArgs a) {
     const int64_t m = blockIdx.x, c = (int64_t)blockIdx.y * 256 + threadIdx.x;
     if (c >= a.ntot) return;
     const int64_t plane = a.M * a.ntot;
-    const float *ws = a.ws + m * a.ntot + c;
+    const float *ws = a.ws + (int64_t)blockIdx.z * a.nsplit * plane + m * a.ntot + c;
     float sum = ws[0];
     for (int s = 1; s < a.nsplit; s++) sum += ws[s * plane];
     int pi = 0;
 #pragma unroll
     for (int i = 1; i < 4; i++) pi += i < a.nprob && c >= a.col0[i];
     float *y = fg_pick(pi, a.prob[0].y, a.prob[1].y, a.prob[2].y, a.prob[3].y);
+    if (a.batched) {
+        const FgSlice z = fg_slice(a, blockIdx.z);
+        y = (float *)((uint8_t *)y + z.i2 * a.y_b2 + z.i3 * a.y_b3);
+    }
     const int64_t ldy = fg_pick(pi, a.prob[0].ldy, a.prob[1].ldy, a.prob[2].ldy, a.prob[3].ldy);
     y[m * ldy + (c - fg_pick(pi, a.col0[0], a.col0[1], a.col0[2], a.col0[3]))] = sum;
 }
@@ -366,7 +397,7 @@ namespace {
 struct FgPlan {
     int tile = 0, bm = 0, bn = 0, nsplit = 1;
     bool pass = false;  // F16: the activations are rounded to fp16 rows in scratch first
-    int64_t ntot = 0;
+    int64_t ntot = 0, grid = 0, rows = 0, slices = 0;  // of one launch: workgroups per slice, rows, slices
 };
 
 // Tiles (BM x BN, K groups) and K splits over workgroups, by the tiles the product has. Measured on MI355X with weights
@@ -378,15 +409,22 @@ struct FgPlan {
 //   F16, N = 2048, K = 6144: M = 512 64 x 64 in two splits 34.4, in one 39.6; M = 133 64 x 64 in four 20.1, 32 x 64 in
 //     one 25.7; M = 28 32 x 32 in four 12.1, in one 20.1
 //   F32, K = 2048, N = 64, M = 256: 16 x 16 7.4, 32 x 32 18.8; K = 3008, N = 1200, M = 396: 32 x 32 40.8, 16 x 16 70.0
+//     (16 x 16: 98 KB, one workgroup per CU, eight waves that share K in stages of 256). Where K is one stage, a second round
+//     of them costs more than the larger tile: K = 128, N = 512, 16 slices of M = 9 7.6, 32 x 32 5.2
 // The mat-vec that these products ran on before takes 8 columns (fewer for K > 2048) at a time: F16 512 x 12288 x 2048
 // 2,604 us, F32 256 x 64 x 2048 356 us.
-FgPlan fg_plan(int type, int nprob, const int64_t *N, int64_t M, int64_t K) {
+// Batch slices share a launch, and their tiles count together. A launch for each slice against one for all, and the
+// mat-vec, which takes every slice of eight columns: F16, N = 512, K = 128: 16 slices of M = 9 64.8 / 5.6 / 6.9 us, 256 of
+// M = 64 1,236 / 31.5 / 201; F32, N = 64, K = 2048, 256 slices of M = 16 2,067 / 48.2 / 202.
+FgPlan fg_plan_rows(const GemmFArgs &g, int64_t M) {
     FgPlan pl;
-    for (int i = 0; i < nprob; i++) pl.ntot += N[i];
-    auto tiles = [&](int bm, int bn) {
+    const int type = g.type;
+    const int64_t K = g.K;
+    for (int i = 0; i < g.nprob; i++) pl.ntot += g.N[i];
+    auto tiles = [&](int bm, int bn) {  // of every slice
         int64_t t = 0;
-        for (int i = 0; i < nprob; i++) t += (N[i] + bn - 1) / bn;
-        return t * ((M + bm - 1) / bm);
+        for (int i = 0; i < g.nprob; i++) t += (g.N[i] + bn - 1) / bn;
+        return t * ((M + bm - 1) / bm) * g.nbatch;
     };
     static constexpr int T16[][3] = {{128, 128, 1}, {64, 128, 1}, {64, 64, 2}, {32, 64, 4}, {32, 32, 4}};
     static constexpr int T32[][3] = {{32, 32, 2}, {16, 16, 8}};
@@ -403,7 +441,7 @@ FgPlan fg_plan(int type, int nprob, const int64_t *N, int64_t M, int64_t K) {
         if (pl.tile == 2 && long_k && t64 > 0) want = std::min<int64_t>(4, 512 / t64);
         if (pl.tile == 4 && t32 > 0 && t32 <= 128) want = std::min<int64_t>(256 / t32, K / 1536);
     } else {
-        pl.tile = tiles(16, 16) <= 512;
+        pl.tile = tiles(16, 16) <= (K > 256 ? 512 : 256);
     }
     const auto &t = type == MX_TYPE_F16 ? T16[pl.tile] : T32[pl.tile];
     pl.bm = t[0];
@@ -413,79 +451,125 @@ FgPlan fg_plan(int type, int nprob, const int64_t *N, int64_t M, int64_t K) {
     want = std::max<int64_t>(1, std::min(want, nst));
     const int64_t per = (nst + want - 1) / want;  // stages of a split; none is left empty
     pl.nsplit = (int)((nst + per - 1) / per);
+    pl.grid = tiles(pl.bm, pl.bn) / g.nbatch * pl.nsplit;
+    pl.rows = M;
     return pl;
 }
 
-size_t fg_act_bytes(const FgPlan &pl, int64_t M, int64_t K) {
-    return pl.pass ? ((size_t)M * (size_t)K * 2 + 255) / 256 * 256 : 0;
+// Bytes of scratch for `slices` slices of a launch: the fp16 rows, and the partial sums.
+size_t fg_act_bytes(const FgPlan &pl, int64_t K, int64_t slices) {
+    return pl.pass ? ((size_t)slices * (size_t)pl.rows * (size_t)K * 2 + 255) / 256 * 256 : 0;
+}
+size_t fg_bytes(const FgPlan &pl, int64_t K, int64_t slices) {
+    return fg_act_bytes(pl, K, slices) +
+           (pl.nsplit > 1 ? (size_t)slices * (size_t)pl.nsplit * (size_t)pl.rows * (size_t)pl.ntot * 4 : 0);
+}
+
+// ... with the rows and the slices of one launch: a grid dimension of fewer than 2^32 threads (HIP's limit; the pass and
+// the reduce have 256 a row), and scratch for as many slices as stay within 64 MB. grid = 0: no launch can have it.
+FgPlan fg_plan(const GemmFArgs &g) {
+    constexpr int64_t ROWS = (int64_t)1 << 22, THREADS = (int64_t)1 << 32, WG = 512, WORK = (int64_t)64 << 20;
+    FgPlan pl = fg_plan_rows(g, std::min(g.M, ROWS));
+    while (pl.grid * WG >= THREADS && pl.rows > 32) pl = fg_plan_rows(g, (pl.rows / 2 + 31) / 32 * 32);
+    if (pl.grid * WG >= THREADS) pl.grid = 0;
+    const size_t one = fg_bytes(pl, g.K, 1);
+    pl.slices = one ? std::max<int64_t>(1, std::min<int64_t>(g.nbatch, WORK / (int64_t)one)) : g.nbatch;
+    return pl;
 }
 
 template <class C>
-hipError_t fg_launch(int64_t grid, const FgArgs &a, hipStream_t s) {
+hipError_t fg_launch(int64_t grid, unsigned slices, const FgArgs &a, hipStream_t s) {
     static const hipError_t attr =
         hipFuncSetAttribute((const void *)k_gemm_f<C>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
     if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL(k_gemm_f<C>, dim3((unsigned)grid), dim3(64 * C::NW), C::LDS, s, a);
+    hipLaunchKernelGGL(k_gemm_f<C>, dim3((unsigned)grid, slices), dim3(64 * C::NW), C::LDS, s, a);
+    return hipGetLastError();
+}
+
+// The rows m0 .. m0 + M (at most pl.rows) of the slices z0 .. z0 + slices.
+hipError_t fg_run(const GemmFArgs &g, const FgPlan &pl, int64_t m0, int64_t M, int64_t z0, unsigned slices,
+                  void *scratch, hipStream_t s) {
+    FgArgs a{};
+    int64_t tiles = 0;
+    for (int i = 0; i < g.nprob; i++) {
+        a.prob[i] = FgProblem{(const uint8_t *)g.w[i], g.N[i], g.y[i] + m0 * g.ldy[i], g.ldy[i]};
+        a.col0[i] = i == 0 ? 0 : a.col0[i - 1] + g.N[i - 1];
+        tiles += (g.N[i] + pl.bn - 1) / pl.bn;
+    }
+    tiles *= (M + pl.bm - 1) / pl.bm;
+    if (tiles == 0) return hipSuccess;
+    a.nprob = g.nprob;
+    a.nsplit = pl.nsplit;
+    a.M = M;
+    a.K = g.K;
+    a.x = (const uint8_t *)g.x + m0 * g.x_nb;
+    a.x_nb = g.x_nb;
+    a.ntot = pl.ntot;
+    a.ws = (float *)((uint8_t *)scratch + fg_act_bytes(pl, g.K, slices));
+    if (g.nbatch > 1) {
+        a.batched = 1;
+        a.z0 = (uint32_t)z0;
+        a.ne2 = (uint32_t)g.ne2;
+        a.r2 = (uint32_t)g.r2;
+        a.r3 = (uint32_t)g.r3;
+        a.x_b2 = g.x_b2;
+        a.x_b3 = g.x_b3;
+        a.w_b2 = g.w_b2;
+        a.w_b3 = g.w_b3;
+        a.y_b2 = g.y_b2;
+        a.y_b3 = g.y_b3;
+    }
+    if (pl.pass) {
+        hipLaunchKernelGGL(k_f16_act, dim3((unsigned)M, (unsigned)((g.K + 2047) / 2048), slices), dim3(256), 0, s,
+                           (const float *)a.x, g.x_nb / 4, g.K, (uint16_t *)scratch, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        a.x = (const uint8_t *)scratch;
+        a.x_nb = 2 * g.K;
+        a.x_b2 = 2 * g.K * M;
+    }
+    const int64_t grid = tiles * pl.nsplit;
+    hipError_t e;
+    if (g.type == MX_TYPE_F16) {
+        switch (pl.tile) {
+            case 0: e = fg_launch<FgCfg<MX_TYPE_F16, 128, 128, 2, 2, 1, 2>>(grid, slices, a, s); break;
+            case 1: e = fg_launch<FgCfg<MX_TYPE_F16, 64, 128, 2, 2, 1, 3>>(grid, slices, a, s); break;
+            case 2: e = fg_launch<FgCfg<MX_TYPE_F16, 64, 64, 2, 2, 2, 2>>(grid, slices, a, s); break;
+            case 3: e = fg_launch<FgCfg<MX_TYPE_F16, 32, 64, 1, 2, 4, 2, true>>(grid, slices, a, s); break;
+            default: e = fg_launch<FgCfg<MX_TYPE_F16, 32, 32, 1, 1, 4, 3, true>>(grid, slices, a, s); break;
+        }
+    } else {
+        e = pl.tile == 0 ? fg_launch<FgCfg<MX_TYPE_F32, 32, 32, 2, 2, 2, 3>>(grid, slices, a, s)
+                         : fg_launch<FgCfg<MX_TYPE_F32, 16, 16, 1, 1, 8, 3>>(grid, slices, a, s);
+    }
+    if (e != hipSuccess || pl.nsplit == 1) return e;
+    hipLaunchKernelGGL(k_fg_reduce, dim3((unsigned)M, (unsigned)((pl.ntot + 255) / 256), slices), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 }  // namespace
 
-bool gemm_f_supported(int type, int64_t M, int64_t K, int64_t x_nb) {
-    if (type != MX_TYPE_F16 && type != MX_TYPE_F32) return false;
+bool gemm_f_supported(const GemmFArgs &g) {
+    if ((g.type != MX_TYPE_F16 && g.type != MX_TYPE_F32) || (g.nprob > 1 && g.nbatch > 1)) return false;
     // a tile's rows within the descriptors' 32-bit offsets
-    return x_nb >= 0 && x_nb < ((int64_t)1 << 24) && K < ((int64_t)1 << 22) && M < ((int64_t)1 << 31);
+    if (g.x_nb < 0 || g.x_nb >= ((int64_t)1 << 24) || g.K >= ((int64_t)1 << 22) || g.M >= ((int64_t)1 << 31)) return false;
+    const FgPlan pl = fg_plan(g);
+    return pl.grid > 0 && (pl.nsplit == 1 || pl.ntot <= 256 * 65535);
 }
 
-size_t gemm_f_scratch_bytes(int type, int nprob, const int64_t *N, int64_t M, int64_t K) {
-    const FgPlan pl = fg_plan(type, nprob, N, M, K);
-    return fg_act_bytes(pl, M, K) + (pl.nsplit > 1 ? (size_t)pl.nsplit * (size_t)M * (size_t)pl.ntot * 4 : 0);
+size_t gemm_f_scratch_bytes(const GemmFArgs &g) {
+    const FgPlan pl = fg_plan(g);
+    return fg_bytes(pl, g.K, pl.slices);
 }
 
-hipError_t launch_gemm_f(int type, int nprob, const void *const *w, const int64_t *N, const float *x, int64_t x_nb,
-                         float *const *y, const int64_t *ldy, int64_t M, int64_t K, void *scratch, hipStream_t s) {
-    const FgPlan pl = fg_plan(type, nprob, N, M, K);
-    FgArgs a{};
-    int64_t tiles = 0;
-    for (int i = 0; i < nprob; i++) {
-        a.prob[i] = FgProblem{(const uint8_t *)w[i], N[i], y[i], ldy[i]};
-        a.col0[i] = i == 0 ? 0 : a.col0[i - 1] + N[i - 1];
-        tiles += (N[i] + pl.bn - 1) / pl.bn;
-    }
-    tiles *= (M + pl.bm - 1) / pl.bm;
-    if (tiles == 0) return hipSuccess;
-    a.nprob = nprob;
-    a.nsplit = pl.nsplit;
-    a.M = M;
-    a.K = K;
-    a.x = (const uint8_t *)x;
-    a.x_nb = x_nb;
-    a.ntot = pl.ntot;
-    a.ws = (float *)((uint8_t *)scratch + fg_act_bytes(pl, M, K));
-    if (pl.pass) {
-        hipLaunchKernelGGL(k_f16_act, dim3((unsigned)M, (unsigned)((K + 2047) / 2048)), dim3(256), 0, s, x, x_nb / 4, K,
-                           (uint16_t *)scratch);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        a.x = (const uint8_t *)scratch;
-        a.x_nb = 2 * K;
-    }
-    const int64_t grid = tiles * pl.nsplit;
-    hipError_t e;
-    if (type == MX_TYPE_F16) {
-        switch (pl.tile) {
-            case 0: e = fg_launch<FgCfg<MX_TYPE_F16, 128, 128, 2, 2, 1, 2>>(grid, a, s); break;
-            case 1: e = fg_launch<FgCfg<MX_TYPE_F16, 64, 128, 2, 2, 1, 3>>(grid, a, s); break;
-            case 2: e = fg_launch<FgCfg<MX_TYPE_F16, 64, 64, 2, 2, 2, 2>>(grid, a, s); break;
-            case 3: e = fg_launch<FgCfg<MX_TYPE_F16, 32, 64, 1, 2, 4, 2, true>>(grid, a, s); break;
-            default: e = fg_launch<FgCfg<MX_TYPE_F16, 32, 32, 1, 1, 4, 3, true>>(grid, a, s); break;
+hipError_t launch_gemm_f(const GemmFArgs &g, void *scratch, hipStream_t s) {
+    const FgPlan pl = fg_plan(g);
+    for (int64_t z0 = 0; z0 < g.nbatch; z0 += pl.slices)
+        for (int64_t m0 = 0; m0 < g.M; m0 += pl.rows) {
+            const hipError_t e = fg_run(g, pl, m0, std::min(pl.rows, g.M - m0), z0,
+                                        (unsigned)std::min(pl.slices, g.nbatch - z0), scratch, s);
+            if (e != hipSuccess) return e;
         }
-    } else {
-        e = pl.tile == 0 ? fg_launch<FgCfg<MX_TYPE_F32, 32, 32, 2, 2, 2, 3>>(grid, a, s)
-                         : fg_launch<FgCfg<MX_TYPE_F32, 16, 16, 1, 1, 8, 3>>(grid, a, s);
-    }
-    if (e != hipSuccess || pl.nsplit == 1) return e;
-    hipLaunchKernelGGL(k_fg_reduce, dim3((unsigned)M, (unsigned)((pl.ntot + 255) / 256)), dim3(256), 0, s, a);
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 }  // namespace mx

@@ -807,33 +807,38 @@ static int gemm_dq_group(mx_backend *be, int n, const mx_tensor *const *src0, co
     return MX_SUCCESS;
 }
 
-// M > 8 on F16 / F32 weights: per batch slice, one launch over every weight sharing src1 (behind the pass that rounds
-// src1 to fp16 for F16 weights on the larger tiles). *done stays false where the product needs scratch that cannot be
-// had now: the mat-vec over groups of columns computes it without any.
+// M > 8 on F16 / F32 weights: one launch over every weight sharing src1 and every batch slice (behind the pass that
+// rounds src1 to fp16 for F16 weights on the larger tiles). *done stays false where the GEMM cannot take the product, or
+// needs scratch that cannot be had now: the mat-vec over groups of columns computes it without any.
 static int gemm_f_group(mx_backend *be, int n, const mx_tensor *const *src0, const mx_tensor *src1,
                         const mx_tensor *const *dst, bool *done) {
     const mx_tensor *w0 = src0[0];
-    const int64_t K = w0->ne[0], M = src1->ne[1];
-    int64_t N[4], ldy[4];
+    mx::GemmFArgs g{};
+    g.type = w0->type;
+    g.nprob = n;
+    g.M = src1->ne[1];
+    g.K = w0->ne[0];
+    g.x = (const float *)src1->data;
+    g.x_nb = (int64_t)src1->nb[1];
     for (int i = 0; i < n; i++) {
-        N[i] = src0[i]->ne[1];
-        ldy[i] = (int64_t)(dst[i]->nb[1] / 4);
+        g.w[i] = src0[i]->data;
+        g.N[i] = src0[i]->ne[1];
+        g.y[i] = (float *)dst[i]->data;
+        g.ldy[i] = (int64_t)(dst[i]->nb[1] / 4);
     }
-    if (!ensure_work(be, mx::gemm_f_scratch_bytes(w0->type, n, N, M, K))) return MX_SUCCESS;
+    g.nbatch = src1->ne[2] * src1->ne[3];
+    g.ne2 = src1->ne[2];
+    g.r2 = src1->ne[2] / w0->ne[2];
+    g.r3 = src1->ne[3] / w0->ne[3];
+    g.x_b2 = (int64_t)src1->nb[2];
+    g.x_b3 = (int64_t)src1->nb[3];
+    g.w_b2 = (int64_t)w0->nb[2];
+    g.w_b3 = (int64_t)w0->nb[3];
+    g.y_b2 = (int64_t)dst[0]->nb[2];
+    g.y_b3 = (int64_t)dst[0]->nb[3];
+    if (!mx::gemm_f_supported(g) || !ensure_work(be, mx::gemm_f_scratch_bytes(g))) return MX_SUCCESS;
     *done = true;
-    const int64_t r2 = src1->ne[2] / w0->ne[2], r3 = src1->ne[3] / w0->ne[3];
-    for (int64_t i13 = 0; i13 < src1->ne[3]; i13++)
-        for (int64_t i12 = 0; i12 < src1->ne[2]; i12++) {
-            const float *x = (const float *)((const uint8_t *)src1->data + i12 * src1->nb[2] + i13 * src1->nb[3]);
-            const void *w[4];
-            float *y[4];
-            for (int i = 0; i < n; i++) {
-                w[i] = (const uint8_t *)src0[i]->data + (i12 / r2) * src0[i]->nb[2] + (i13 / r3) * src0[i]->nb[3];
-                y[i] = (float *)((uint8_t *)dst[i]->data + i12 * dst[i]->nb[2] + i13 * dst[i]->nb[3]);
-            }
-            HIP_OK(mx::launch_gemm_f(w0->type, n, w, N, x, (int64_t)src1->nb[1], y, ldy, M, K, be->work, be->stream),
-                   "GEMM launch");
-        }
+    HIP_OK(mx::launch_gemm_f(g, be->work, be->stream), "GEMM launch");
     return MX_SUCCESS;
 }
 
@@ -884,7 +889,7 @@ static int matvec_group(mx_backend *be, int n, const mx_tensor *const *src0, con
         if (fits && mx::gemm_dq_supported(a.type, M, a.K)) return gemm_dq_group(be, n, src0, src1, dst);
         if (a.type == MX_TYPE_Q4_K && a.K % 256 == 0) return gemm_q4k_group(be, n, src0, src1, dst);
         if (mx::gemm_kq_supported(a.type, a.K)) return gemm_kq_group(be, n, src0, src1, dst);
-        if (mx::gemm_f_supported(a.type, M, a.K, (int64_t)src1->nb[1])) {
+        if (a.type == MX_TYPE_F16 || a.type == MX_TYPE_F32) {
             bool done = false;
             const int rc = gemm_f_group(be, n, src0, src1, dst, &done);
             if (rc || done) return rc;

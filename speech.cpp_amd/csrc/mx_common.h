@@ -198,13 +198,25 @@ hipError_t launch_matvec(const MatvecArgs &a, hipStream_t s);
 // The same products on F16 / F32 weights in ggml's row-major layout (prob[i].w.p0 = the weight's data; K % 8 == 0 for
 // F16, K % 4 == 0 for F32; no ids mode).
 hipError_t launch_matvec_f(const MatvecArgs &a, hipStream_t s);
-// Prefill GEMM on F16 / F32 weights (M > 8): up to four weights sharing the activations x (M rows, x_nb bytes apart).
-// The scratch (gemm_f_scratch_bytes) holds the activations rounded to fp16 for F16 weights, and the partial sums where
-// K is split over workgroups.
-bool gemm_f_supported(int type, int64_t M, int64_t K, int64_t x_nb);
-size_t gemm_f_scratch_bytes(int type, int nprob, const int64_t *N, int64_t M, int64_t K);
-hipError_t launch_gemm_f(int type, int nprob, const void *const *w, const int64_t *N, const float *x, int64_t x_nb,
-                         float *const *y, const int64_t *ldy, int64_t M, int64_t K, void *scratch, hipStream_t s);
+// Prefill GEMM on F16 / F32 weights (M > 8): up to four weights sharing the activations x (M rows, x_nb bytes apart), or
+// one weight over nbatch slices (ne2 of them along axis 2, the rest along axis 3; slice (i2, i3) meets matrix (i2 / r2,
+// i3 / r3)). The scratch (gemm_f_scratch_bytes) holds the activations rounded to fp16 for F16 weights, and the partial
+// sums where K is split over workgroups.
+struct GemmFArgs {
+    int type, nprob;
+    int64_t M, K;
+    const void *w[4];
+    int64_t N[4];
+    const float *x;
+    int64_t x_nb;
+    float *y[4];
+    int64_t ldy[4];                              // floats between rows
+    int64_t nbatch, ne2, r2, r3;
+    int64_t x_b2, x_b3, w_b2, w_b3, y_b2, y_b3;  // bytes between slices (matrices of w)
+};
+bool gemm_f_supported(const GemmFArgs &g);
+size_t gemm_f_scratch_bytes(const GemmFArgs &g);
+hipError_t launch_gemm_f(const GemmFArgs &g, void *scratch, hipStream_t s);
 
 // Prefill GEMM on int8 MFMA (Q8_0, M > 8): launch_gemm_quant writes the activations as Q8_0 (int8 quants and fp32
 // block scales) at the start of `scratch`, launch_gemm runs up to four weights sharing them in one launch (plus a

@@ -88,6 +88,62 @@ def test_batches(mx, be, tname):
         check(y[i], w64[(i // 2) * N:(i // 2 + 1) * N], x64[i * M:(i + 1) * M])
 
 
+@pytest.mark.parametrize("tname", ["F16", "F32"])
+@pytest.mark.parametrize("M,N,K,slices,r", [
+    (9, 33, 64, (24, 3), (2, 3)),        # a tile or two a slice, both axes, broadcast along both
+    (40, 200, 4608, (5, 1), (5, 1)),     # K split: one matrix to every slice
+    (130, 260, 4104, (3, 2), (1, 2)),    # K split or the fp16 pass
+    (300, 400, 136, (40, 1), (1, 1)),    # the fp16 pass over every slice
+    (2100, 8, 4096, (4, 1), (2, 1)),     # fp16 rows of 17 MB a slice: more than a launch's scratch holds
+])
+def test_slices_share_launches(mx, tname, M, N, K, slices, r):
+    """However many slices a product has, it takes a few launches (counted in a recording): slices with gaps between them,
+    against double precision; the gaps stay as they were."""
+    be = mx.Backend(0)
+    t, (n2, n3), (r2, r3) = getattr(mx, tname), slices, r
+    m2, m3 = n2 // r2, n3 // r3
+    w, x, w64, x64 = data(mx, t, N * m2 * m3, K, M * n2 * n3, N + K)
+    W = upload(mx, be, t, (K, N, m2, m3), w)
+    xg = np.zeros((n3, n2, M + 3, K), np.float32)  # three rows between slices
+    xg[:, :, :M] = x.reshape(n3, n2, M, K)
+    yg = np.full((n3, n2, M + 2, N + 4), 7.0, np.float32)
+    Xb, Yb = be.tensor(mx.F32, (K, M + 3, n2, n3), xg), be.tensor(mx.F32, (N + 4, M + 2, n2, n3), yg)
+    X = Xb.view((K, M, n2, n3), (4, 4 * K, 4 * K * (M + 3), 4 * K * (M + 3) * n2))
+    Y = Yb.view((N, M, n2, n3), (4, 4 * (N + 4), 4 * (N + 4) * (M + 2), 4 * (N + 4) * (M + 2) * n2))
+    be.mul_mat(W, X, Y)
+    be.sync()
+    got = Yb.numpy()
+    for i3 in range(n3):
+        for i2 in range(n2):
+            z, m = i3 * n2 + i2, (i3 // r3) * m2 + i2 // r2
+            check(got[i3, i2, :M, :N], w64[m * N:(m + 1) * N], x64[z * M:(z + 1) * M])
+    assert np.all(got[:, :, M:] == 7.0) and np.all(got[:, :, :, N:] == 7.0)
+    be.graph_begin()
+    be.mul_mat(W, X, Y)
+    g = be.graph_end()
+    assert be.graph_nodes(g) <= 6  # pass, product, reduce; twice where the scratch holds some of the slices
+    Yb.set(yg)
+    be.graph_launch(g)
+    be.sync()
+    assert np.array_equal(Yb.numpy(), got)
+    be.graph_free(g)
+    del W, X, Y, Xb, Yb
+    be.close()
+
+
+@pytest.mark.parametrize("tname", ["F16", "F32"])
+def test_more_rows_than_a_grid_has(mx, be, tname):
+    """2^24 rows and some: a grid of one workgroup of 256 to a row is refused (2^32 threads). Small integers: exact."""
+    M, N, K = (1 << 24) + 40, 2, 8
+    g = RNG(8)
+    w = g.integers(-8, 8, (N, K)).astype(np.float16 if tname == "F16" else np.float32)
+    x = g.integers(-8, 8, (M, K)).astype(np.float32)
+    W, X, Y = upload(mx, be, getattr(mx, tname), (K, N), w), be.tensor(mx.F32, (K, M), x), be.tensor(mx.F32, (N, M))
+    be.mul_mat(W, X, Y)
+    be.sync()
+    assert np.array_equal(Y.numpy().reshape(M, N), x @ w.astype(np.float32).T)
+
+
 @pytest.mark.parametrize("side", ["weights", "activations"])
 def test_subnormal_halves(mx, be, side):
     """fp16 subnormals count in full: times small integers every sum is a multiple of 2^-24 below 2^-9, exact in fp32."""
