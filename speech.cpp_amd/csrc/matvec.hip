@@ -7,6 +7,7 @@
 #include "mx_device.h"
 #include "mx_dot.h"
 
+#include <algorithm>
 #include <cstdlib>
 
 namespace mx {
@@ -16,23 +17,18 @@ __device__ __forceinline__ MatvecProblem pick_problem(const MatvecArgs &a, int i
     return i == 0 ? a.prob[0] : (i == 1 ? a.prob[1] : (i == 2 ? a.prob[2] : a.prob[3]));
 }
 
-// The most threads of a workgroup. Every workgroup quantizes all of its columns, so the more there are the more rows
-// should share that: eight waves from two columns on (four waves: 2048 + 1024 + 1024 Q8_0 rows of K = 2048, five columns
-// behind a norm, 12.0 us; eight 7.7; Q6_K, 2048 rows of K = 6144, eight columns 26.7 and 17.2). Q5_K keeps four: its dots
-// take more registers than eight waves leave. mv_fixed: launch_nc always takes that many.
-template <int TYPE, int NC>
-__host__ __device__ constexpr int mv_threads() { return NC >= 2 && TYPE != MX_TYPE_Q5_K ? 512 : 256; }
-template <int TYPE, int NC>
-__host__ __device__ constexpr bool mv_fixed() { return NC == 1 || TYPE == MX_TYPE_Q8_0 || TYPE == MX_TYPE_Q5_K; }
-// ... and whether a workgroup goes on to further rows with the columns it has quantized.
-template <int NC>
-__host__ __device__ constexpr bool mv_loops() { return NC >= 2; }
-// A workgroup's waves; the elements of a column it handles at once are 256 a wave (a float4 a thread). Below, the float4s
-// of each column every thread loads ahead of the weights (elements PIECE i + 4 tid, i < XPRE).
-template <int TYPE, int NC>
-__device__ __forceinline__ int mv_waves() {
-    return mv_fixed<TYPE, NC>() ? mv_threads<TYPE, NC>() / 64 : (int)blockDim.x / 64;
+// The two shapes of a workgroup. Narrow: four waves, one set of rows. Wide, from two columns on: eight waves (Q5_K four: its
+// dots take more registers than eight waves leave) that go on to further rows with the columns they have quantized, which
+// every workgroup does for itself. Wide costs registers, so where the columns are soon quantized narrow is faster; mv_wide
+// picks, mv_narrow says which narrow kernels there are.
+template <int TYPE, bool WIDE>
+__host__ __device__ constexpr int mv_waves() { return WIDE && TYPE != MX_TYPE_Q5_K ? 8 : 4; }
+template <int TYPE, int NC, bool FUSED>
+constexpr bool mv_narrow() {
+    return NC == 1 || (TYPE == MX_TYPE_Q5_K && NC <= 4) || ((TYPE == MX_TYPE_Q4_K || TYPE == MX_TYPE_Q6_K) && (!FUSED || NC <= 5));
 }
+// The elements of a column that a workgroup handles at once (a PIECE) are 256 a wave, a float4 a thread. Every thread
+// loads the first XPRE float4s of each column (elements PIECE i + 4 tid) ahead of the weights.
 template <int NC>
 __host__ __device__ constexpr int xpre() { return NC == 1 ? 4 : (NC == 2 ? 2 : 1); }
 
@@ -80,17 +76,16 @@ __device__ __forceinline__ float4 load_x4(const float *xc, int e, int K) {
 // then mul(rms_norm(x, eps), norm_w) when norm_w is set -- the squares (rounded to float) summed in double over the
 // workgroup, the mean rounded to float, x * (1 / sqrtf(mean + eps)) then times the weight, as the separate ops round
 // -- and is quantized. Pieces past the preloaded ones are read again after the sum.
-template <int TYPE, int NC>
+template <int TYPE, int NC, int NW>
 __device__ __forceinline__ void fused_prologue(const MatvecArgs &a, const float *x, int xi12, int i13,
                                                float4 (&xr)[NC][xpre<NC>()], const float4 (&br)[NC][xpre<NC>()],
                                                const float4 (&wr)[xpre<NC>()], int8_t *xq, float *xd, int *xbs) {
     constexpr int XP = xpre<NC>();
-    const int PIECE = 256 * mv_waves<TYPE, NC>();
+    constexpr int PIECE = 256 * NW;
     constexpr int XDB = TYPE == MX_TYPE_Q8_0 ? 32 : 256;
     const int K = (int)a.K;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int MW = mv_threads<TYPE, NC>() / 64;
-    __shared__ double red[NC][MW];
+    __shared__ double red[NC][NW];
     const float *gb = a.glu_b ? a.glu_b + xi12 * a.x_b2 + i13 * a.x_b3 : nullptr;
     // glu of one loaded piece; the preloaded pieces' second operands came in with x (br)
     auto piece_b = [&](float4 v, float4 b) -> float4 {
@@ -142,14 +137,13 @@ __device__ __forceinline__ void fused_prologue(const MatvecArgs &a, const float 
         for (int c = 0; c < NC; c++) {
             ss[c] = wave_sum_d(ss[c]);
             if (lane == 0) red[c][wave] = ss[c];
-            if (!mv_fixed<TYPE, NC>() && lane == 0 && PIECE < 256 * MW) red[c][MW / 2 + wave] = 0.0;  // four waves of eight
         }
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             double tot = red[c][0];
 #pragma unroll
-            for (int w = 1; w < MW; w++) tot += red[c][w];
+            for (int w = 1; w < NW; w++) tot += red[c][w];
             const float mean = (float)(tot / (double)K);
             scale[c] = 1.0f / sqrtf(mean + a.norm_eps);
         }
@@ -183,11 +177,11 @@ __device__ __forceinline__ void fused_prologue(const MatvecArgs &a, const float 
 
 // The plain prologue: every column quantized into LDS, the preloaded pieces first, the others piece by piece with all
 // columns' loads in flight.
-template <int TYPE, int NC>
+template <int TYPE, int NC, int NW>
 __device__ __forceinline__ void plain_prologue(const MatvecArgs &a, const float *x, const float4 (&xr)[NC][xpre<NC>()],
                                                int8_t *xq, float *xd, int *xbs) {
     constexpr int XP = xpre<NC>();
-    const int PIECE = 256 * mv_waves<TYPE, NC>();
+    constexpr int PIECE = 256 * NW;
     constexpr int XDB = TYPE == MX_TYPE_Q8_0 ? 32 : 256;
     const int K = (int)a.K;
     auto quantize = [&](int c, int base, float4 v) {
@@ -209,10 +203,10 @@ __device__ __forceinline__ void plain_prologue(const MatvecArgs &a, const float 
 
 // FUSED: the instantiation that reads the fused operands (norm weight, SwiGLU input, residual); the plain one is
 // compiled without them, so products with no fusion keep their smaller register footprint.
-template <int TYPE, int NC, int LPR, bool FUSED>
-__global__ __launch_bounds__((mv_threads<TYPE, NC>())) void k_matvec(MatvecArgs a) {
+template <int TYPE, int NC, int LPR, bool FUSED, bool WIDE>
+__global__ __launch_bounds__((64 * mv_waves<TYPE, WIDE>())) void k_matvec(MatvecArgs a) {
     extern __shared__ __align__(16) uint8_t smem[];
-    const int NW = mv_waves<TYPE, NC>();
+    constexpr int NW = mv_waves<TYPE, WIDE>();
     const int K = (int)a.K;
     const int tid = threadIdx.x;
     // The argument block's fields on the way to the first weight load, requested together into scalar registers:
@@ -254,7 +248,7 @@ __global__ __launch_bounds__((mv_threads<TYPE, NC>())) void k_matvec(MatvecArgs 
     // The activation loads go first: x -> quantization -> LDS is the prologue's critical path, and the memory counter
     // retires loads in order, so waiting for x then does not wait for the weight loads issued after it.
     constexpr int XP = xpre<NC>();
-    const int PIECE = 256 * mv_waves<TYPE, NC>();
+    constexpr int PIECE = 256 * NW;
     float4 xr[NC][XP];
 #pragma unroll
     for (int c = 0; c < NC; c++)
@@ -309,12 +303,12 @@ __global__ __launch_bounds__((mv_threads<TYPE, NC>())) void k_matvec(MatvecArgs 
     int *xbs = (int *)(xd + NC * (K / XDB));
     if constexpr (FUSED) {
         if (a.glu_b || a.norm_w) {  // uniform: the fused prologue
-            fused_prologue<TYPE, NC>(a, x, xi12, i13, xr, br, wr, xq, xd, xbs);
+            fused_prologue<TYPE, NC, NW>(a, x, xi12, i13, xr, br, wr, xq, xd, xbs);
         } else {
-            plain_prologue<TYPE, NC>(a, x, xr, xq, xd, xbs);
+            plain_prologue<TYPE, NC, NW>(a, x, xr, xq, xd, xbs);
         }
     } else {
-        plain_prologue<TYPE, NC>(a, x, xr, xq, xd, xbs);
+        plain_prologue<TYPE, NC, NW>(a, x, xr, xq, xd, xbs);
     }
     __syncthreads();
     if (!has_row) return;  // whole LPR-lane groups leave together; no barrier follows
@@ -338,7 +332,7 @@ __global__ __launch_bounds__((mv_threads<TYPE, NC>())) void k_matvec(MatvecArgs 
                 chunk_dot<TYPE, NC, false>(p.w, grow, K, c, xq, xd, xbs, NC, acc);
         }
         const int64_t next = row + (int64_t)gridDim.x * (NW * G);
-        const bool more = mv_loops<NC>() && next < p.N;
+        const bool more = WIDE && next < p.N;
         if (more) {  // the next rows' first chunks, ahead of this row's reduction and store
             grow = row00 + next;
 #pragma unroll
@@ -378,54 +372,95 @@ static int pick_lpr(int64_t nchunks, int preload, int forced) {
     return lpr;
 }
 
-template <int TYPE, int NC, int LPR>
-static hipError_t launch_one(const MatvecArgs &a, int64_t maxN, int nt, size_t lds, hipStream_t s) {
-    constexpr int G = 64 / LPR;
-    const int R = nt / 64 * G;  // rows of a workgroup
-    bool fused = a.glu_b || a.norm_w;
-    for (int i = 0; i < a.nprob; i++) fused = fused || a.prob[i].res;
-    int64_t groups = (maxN + R - 1) / R;
-    if (mv_loops<NC>()) {
-        // Workgroups that go on to further rows, once there are more than the chip holds at a time: a fused kernel's
-        // registers leave room for one eight-wave workgroup per CU, a plain one's for two. Q8_0, five columns: gate and
-        // up of 2 x 6144 rows, K = 2048, behind a norm, as 256 / 384 / 768 workgroups 11.2 / 16.8 / 19.3 us; 151,936
-        // rows of K = 1024 as 256 / 512 / 768 / 4748 37.1 / 31.6 / 34.2 / 44.2 us.
-        int64_t total = 0;
-        for (int i = 0; i < a.nprob; i++) total += (a.prob[i].N + R - 1) / R;
-        const int64_t cap = fused ? 256 : 512, per = (total * a.nbatch + cap - 1) / cap;
-        groups = (groups + per - 1) / per;
+// The wide workgroups to launch at most: as many as the chip holds at a time by the kernel's registers and by LDS, behind a
+// fused prologue one to a CU (2 x 6144 Q8_0 rows of K = 2048, four columns: 256 workgroups 10.2 us, 512 12.0).
+template <int TYPE, int NC, int LPR, bool FUSED>
+static int64_t mv_most(size_t lds) {
+    if constexpr (FUSED) return 256;
+    static const int regs = [] {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void *)k_matvec<TYPE, NC, LPR, FUSED, true>,
+                                                         64 * mv_waves<TYPE, true>(), 0) != hipSuccess)
+            (void)hipGetLastError();
+        return std::max(n, 1);
+    }();
+    return 256 * std::max<int64_t>(1, std::min<int64_t>(regs, 160 * 1024 / (int64_t)(lds + 1024)));
+}
+
+static int64_t mv_groups(const MatvecArgs &a, int64_t rows) {  // workgroups of so many rows that hold every problem
+    int64_t n = 0;
+    for (int i = 0; i < a.nprob; i++) n += (a.prob[i].N + rows - 1) / rows;
+    return n * a.nbatch;
+}
+
+// Wide or narrow (us, narrow / wide):
+//   Q4_K, Q6_K. A wave quantizes whole super-blocks, so only four of eight would up to K = 1024. Q4_K, 2 x 3072 rows of K =
+//     1024, two columns 4.6 / 4.7, behind a norm 6.0 / 6.2 (eight columns 12.2 / 12.0); 1024 rows, four columns 5.3 / 6.1;
+//     16,384 rows, four columns 8.6 / 7.9. Q6_K, 2 x 6144 rows of K = 1024, eight columns 11.5 / 11.8, behind a norm
+//     27.2 / 15.0 (narrow takes 256 registers there). K = 2048, 2 x 3072 rows, two columns: Q4_K 5.8 / 5.0, Q6_K 7.1 / 6.4.
+//   Q5_K. One wide workgroup fits a CU (256 registers), two or three narrow ones up to four columns: 2 x 6144 rows of K =
+//     2048, two columns 9.2 / 10.8, three 13.3 / 12.8, four 15.4 / 14.8, five (narrow 256 registers too) 25.6 / 16.2. A
+//     second round that is half empty costs the wide form most: 2 x 3072 rows, four columns 9.9 / 11.5.
+template <int TYPE, int NC, bool FUSED>
+static bool mv_wide(const MatvecArgs &a, int lpr) {
+    if constexpr (!mv_narrow<TYPE, NC, FUSED>()) return true;
+    if (NC == 1) return false;
+    if (TYPE == MX_TYPE_Q5_K) {
+        const int64_t groups = mv_groups(a, 4 * (64 / lpr)), cap = 256;
+        if (groups <= cap) return FUSED || 2 * groups > cap;
+        return NC == 2 ? a.K >= 4096 : groups >= 2 * cap;
     }
-    dim3 grid((unsigned)groups, (unsigned)a.nprob, (unsigned)a.nbatch);
-    if (fused) hipLaunchKernelGGL((k_matvec<TYPE, NC, LPR, true>), grid, dim3((unsigned)nt), lds, s, a);
-    else hipLaunchKernelGGL((k_matvec<TYPE, NC, LPR, false>), grid, dim3((unsigned)nt), lds, s, a);
-    return hipGetLastError();
+    return a.K > 1024 || mv_groups(a, 1) >= 16384;
+}
+
+template <int TYPE, int NC, int LPR, bool FUSED, bool WIDE>
+static hipError_t launch_one(const MatvecArgs &a, int64_t maxN, size_t lds, hipStream_t s) {
+    if constexpr (WIDE ? NC >= 2 : mv_narrow<TYPE, NC, FUSED>()) {
+        constexpr int NW = mv_waves<TYPE, WIDE>(), R = NW * (64 / LPR);  // rows of a workgroup
+        int64_t groups = (maxN + R - 1) / R;
+        if constexpr (WIDE) {
+            // They go on to further rows once there are more than that. Q8_0, five columns: gate and up of 2 x 6144 rows, K =
+            // 2048, behind a norm, as 256 / 384 / 768 workgroups 11.2 / 16.8 / 19.3 us; 151,936 rows of K = 1024 (two fit a
+            // CU) as 256 / 512 / 768 / 4748 37.1 / 31.6 / 34.2 / 44.2 us. Q6_K, 37,984 rows of K = 2048, four columns (one
+            // fits), as 256 / 512 21.8 / 27.0 us.
+            const int64_t cap = mv_most<TYPE, NC, LPR, FUSED>(lds), per = (mv_groups(a, R) + cap - 1) / cap;
+            groups = (groups + per - 1) / per;
+        }
+        const dim3 grid((unsigned)groups, (unsigned)a.nprob, (unsigned)a.nbatch);
+        hipLaunchKernelGGL((k_matvec<TYPE, NC, LPR, FUSED, WIDE>), grid, dim3(64 * NW), lds, s, a);
+        return hipGetLastError();
+    }
+    return hipErrorInvalidValue;  // (mv_wide picks what there is)
+}
+
+template <int TYPE, int NC, bool FUSED>
+static hipError_t launch_lpr(const MatvecArgs &a, int64_t maxN, size_t lds, hipStream_t s) {
+    const int64_t nchunks = a.K / chunk_elems<TYPE>();
+    int lpr = pick_lpr(nchunks, preload_of<TYPE>(), a.lpr);
+    const bool wide = mv_wide<TYPE, NC, FUSED>(a, lpr);
+    if (wide && mv_waves<TYPE, true>() > 4 && a.lpr == 0)
+        // eight waves: fewer rows each rather than CUs left idle, while every lane has a chunk
+        while (lpr < 64 && nchunks >= 2 * lpr && mv_groups(a, 512 / lpr) < 128) lpr *= 2;
+    switch (lpr) {
+        case 16:
+            return wide ? launch_one<TYPE, NC, 16, FUSED, true>(a, maxN, lds, s) : launch_one<TYPE, NC, 16, FUSED, false>(a, maxN, lds, s);
+        case 32:
+            return wide ? launch_one<TYPE, NC, 32, FUSED, true>(a, maxN, lds, s) : launch_one<TYPE, NC, 32, FUSED, false>(a, maxN, lds, s);
+        default:
+            return wide ? launch_one<TYPE, NC, 64, FUSED, true>(a, maxN, lds, s) : launch_one<TYPE, NC, 64, FUSED, false>(a, maxN, lds, s);
+    }
 }
 
 template <int TYPE, int NC>
 static hipError_t launch_nc(const MatvecArgs &a, int64_t maxN, size_t lds, hipStream_t s) {
-    const int64_t nchunks = a.K / chunk_elems<TYPE>();
-    int lpr = pick_lpr(nchunks, preload_of<TYPE>(), a.lpr);
-    // Four waves for K-quants of at most 1024 elements a row: a wave quantizes whole super-blocks, so that only four of
-    // eight would (Q6_K, 2 x 1024 rows, two columns behind a norm 5.7 us against 6.2).
-    const int nt = !mv_fixed<TYPE, NC>() && a.K <= 1024 ? 256 : mv_threads<TYPE, NC>();
-    if (nt > 256 && a.lpr == 0) {  // eight waves: fewer rows each rather than CUs left idle, while every lane has a chunk
-        auto groups = [&](int l) {
-            const int64_t rows = nt / l;
-            int64_t n = 0;
-            for (int i = 0; i < a.nprob; i++) n += (a.prob[i].N + rows - 1) / rows;
-            return n * a.nbatch;
-        };
-        while (lpr < 64 && nchunks >= 2 * lpr && groups(lpr) < 128) lpr *= 2;
-    }
-    switch (lpr) {
-        case 16: return launch_one<TYPE, NC, 16>(a, maxN, nt, lds, s);
-        case 32: return launch_one<TYPE, NC, 32>(a, maxN, nt, lds, s);
-        default: return launch_one<TYPE, NC, 64>(a, maxN, nt, lds, s);
-    }
+    bool fused = a.glu_b || a.norm_w;
+    for (int i = 0; i < a.nprob; i++) fused = fused || a.prob[i].res;
+    return fused ? launch_lpr<TYPE, NC, true>(a, maxN, lds, s) : launch_lpr<TYPE, NC, false>(a, maxN, lds, s);
 }
 
 template <int TYPE>
-static hipError_t launch_type(const MatvecArgs &a, int64_t maxN, size_t lds, hipStream_t s) {
+hipError_t launch_matvec_q(const MatvecArgs &a, int64_t maxN, hipStream_t s) {
+    const size_t lds = act_lds_bytes(TYPE, a.K, a.ncols);
     switch (a.ncols) {
         case 1: return launch_nc<TYPE, 1>(a, maxN, lds, s);
         case 2: return launch_nc<TYPE, 2>(a, maxN, lds, s);
@@ -439,19 +474,6 @@ static hipError_t launch_type(const MatvecArgs &a, int64_t maxN, size_t lds, hip
     }
 }
 
-hipError_t launch_matvec(const MatvecArgs &a, hipStream_t s) {
-    int64_t maxN = 0;
-    for (int i = 0; i < a.nprob; i++) maxN = a.prob[i].N > maxN ? a.prob[i].N : maxN;
-    if (maxN == 0) return hipSuccess;
-    if (a.type == MX_TYPE_F16 || a.type == MX_TYPE_F32) return launch_matvec_f(a, s);
-    const size_t lds = act_lds_bytes(a.type, a.K, a.ncols);
-    switch (a.type) {
-        case MX_TYPE_Q8_0: return launch_type<MX_TYPE_Q8_0>(a, maxN, lds, s);
-        case MX_TYPE_Q4_K: return launch_type<MX_TYPE_Q4_K>(a, maxN, lds, s);
-        case MX_TYPE_Q5_K: return launch_type<MX_TYPE_Q5_K>(a, maxN, lds, s);
-        case MX_TYPE_Q6_K: return launch_type<MX_TYPE_Q6_K>(a, maxN, lds, s);
-        default: return hipErrorInvalidValue;
-    }
-}
+template hipError_t launch_matvec_q<MX_MV_TYPE>(const MatvecArgs &a, int64_t maxN, hipStream_t s);
 
 }  // namespace mx

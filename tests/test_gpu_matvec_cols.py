@@ -1,5 +1,5 @@
-"""Products of 1 to 8 columns on quantized weights (the mat-vec: eight waves a workgroup and workgroups that go on to
-further rows from two columns on), and the quantizers' divisions, on MI355X against the oracle.
+"""Products of 1 to 8 columns on quantized weights (the mat-vec: four waves and one set of rows a workgroup, or, from two
+columns on, eight waves that go on to further rows), and the quantizers' divisions, on MI355X against the oracle.
 
 The bound of a product: the kernels sum the oracle's exact block integers, K / 32 scaled terms in fp32 in another order
 (at most 192 here), so about sqrt(192) * 2^-24 = 8e-7 of a row's largest output; 2e-5 would still show a lost term. Behind
@@ -34,6 +34,23 @@ def test_columns(mx, be, t, M, N, K):
     be.mul_mat(W, X, Y)
     be.sync()
     assert rel_err(Y.numpy().reshape(M, N), O.mul_mat(t, w, x)) <= 2e-5
+
+
+# either side of the lines between the two shapes: 16,384 rows up to K = 1024 and past it; Q5_K (16 rows a workgroup, 4 at
+# K = 4096) half a chip of workgroups, a chip, two, with M <= 4
+@pytest.mark.parametrize("t", [O.TYPE_Q4_K, O.TYPE_Q5_K, O.TYPE_Q6_K], ids=lambda t: NAMES[t])
+@pytest.mark.parametrize("fused", [False, True], ids=["plain", "residual"])
+@pytest.mark.parametrize("M", [2, 4, 6])
+@pytest.mark.parametrize("N,K", [(16383, 256), (16384, 512), (2049, 256), (4097, 256), (8193, 256), (1030, 4096)])
+def test_shape_of_a_workgroup(mx, be, t, fused, M, N, K):
+    w, x, r = weights(t, N, K, 5 + N), O.fill_normal(7 + M, M, K), O.fill_normal(3, M, N)
+    W, X, Y = be.tensor(t, (K, N), w), be.tensor(mx.F32, (K, M), x), be.tensor(mx.F32, (N, M), r)
+    if fused:
+        be.mul_mat_fused([W], X, [Y], residual=[Y])
+    else:
+        be.mul_mat(W, X, Y)
+    be.sync()
+    assert rel_err(Y.numpy().reshape(M, N) - (r if fused else 0), O.mul_mat(t, w, x)) <= 2e-5
 
 
 @TYPES
