@@ -767,7 +767,8 @@ hipError_t launch_rms_norm(const RowsArgs &a, float eps, const float *w, hipStre
     if (a.nrows == 0) return hipSuccess;
     const bool al = a.ne0 % 4 == 0 && vec4(w, 0) && vec4(a.src, a.s_nb1) && vec4(a.src, a.s_nb2) && vec4(a.src, a.s_nb3) &&
                     vec4(a.dst, a.d_nb1) && vec4(a.dst, a.d_nb2) && vec4(a.dst, a.d_nb3);
-    if (al && a.ne0 >= NORM_MIN && a.ne0 <= NORM_MAX && a.nrows < ((int64_t)1 << 31)) {
+    // (a workgroup of 256 to a row: HIP refuses a grid of 2^32 threads; the wave form has a wave to a row)
+    if (al && a.ne0 >= NORM_MIN && a.ne0 <= NORM_MAX && a.nrows < ((int64_t)1 << 24)) {
         const dim3 g((unsigned)a.nrows);
         if (a.ne0 <= 1024) hipLaunchKernelGGL(k_rms_norm_wide<1>, g, dim3(256), 0, s, a, eps, w);
         else if (a.ne0 <= 2048) hipLaunchKernelGGL(k_rms_norm_wide<2>, g, dim3(256), 0, s, a, eps, w);

@@ -116,3 +116,24 @@ def test_qk_norm_rope_kv_rows(mx, be, nq, nkv, rows):
         results.append([t.get_bytes() for t in (out, kc, vc)])
     for a, b in zip(*results):
         assert np.array_equal(a, b)
+
+
+def test_norm_of_more_rows_than_a_grid_has(mx, be):
+    """2^24 rows of 1024 floats (64 GiB, in place): a workgroup of 256 to a row would be a grid of 2^32 threads, which is
+    refused. The first rows, the last ones and some between."""
+    n, rows = 1024, 1 << 24
+    try:
+        X = be.tensor(mx.F32, (n, rows))
+    except mx.MxError as e:
+        pytest.skip(f"no 64 GiB on the device: {e}")
+    at = [0, 1, 2, 3, (1 << 22) + 5, (1 << 23) - 1, rows - 2, rows - 1]
+    x = np.random.default_rng(4).standard_normal((len(at), n)).astype(np.float32)
+    for r, v in zip(at, x):
+        X.set(v, 4 * n * r)
+    be.rms_norm(X, X, 1e-6)
+    be.sync()
+    got = np.stack([X.get_bytes(4 * n * r, 4 * n).view(np.float32) for r in at])
+    x64 = x.astype(np.float64)
+    want = x64 / np.sqrt((x64 ** 2).mean(1, keepdims=True) + 1e-6)
+    assert np.all(np.abs(got - want) <= 2.0 ** -22 * np.abs(want))
+    X.free()
