@@ -82,74 +82,6 @@ __device__ __forceinline__ v2h fm_halves(float a, float b, float s) {
     return h;
 }
 
-// One wave's sums of head h, row i over a split's positions, in fp32 and over the positions that the row sees alone
-// (qs [D], ps [64]: LDS of its own). k_fa_mfma's second form where values are infinities or NaN, so small rather than fast.
-template <int D>
-__device__ __forceinline__ void fa_row_alone(const FaArgs &a, int64_t split, int64_t h, int64_t i, int lane, float *qs,
-                                             float *ps) {
-    constexpr int DL = D / 64, NV = 16;  // channels per lane; value rows in flight
-    auto own = []() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
-    const int64_t hk = h / a.gqa, j0 = split * a.split_len, j1 = min(a.n_kv, j0 + a.split_len);
-    const uint8_t *kb = (const uint8_t *)a.k + hk * a.k_nb2, *vb = (const uint8_t *)a.v + hk * a.v_nb2;
-    const uint16_t *mrow = a.mask ? (const uint16_t *)((const uint8_t *)a.mask + i * a.m_nb1) : nullptr;
-    const float *q = (const float *)((const uint8_t *)a.q + i * a.q_nb1 + h * a.q_nb2);
-    own();
-#pragma unroll
-    for (int c = 0; c < DL; c++) qs[64 * c + lane] = h2f(f2h(q[64 * c + lane]));
-    own();
-    float M = -INFINITY, S = 0.0f, acc[DL] = {};
-    for (int64_t base = j0; base < j1; base += 64) {
-        const int64_t j = base + lane;
-        const float m = j < j1 ? (mrow ? h2f(mrow[j]) : 0.0f) : -INFINITY;
-        float s = -INFINITY;
-        if (m != -INFINITY) {
-            const v8h *kr = (const v8h *)(kb + j * a.k_nb1);
-            float dot = 0.0f;
-#pragma unroll 4
-            for (int c = 0; c < D / 8; c++) {
-                const v8h w = kr[c];
-#pragma unroll
-                for (int e = 0; e < 8; e++) dot = fmaf((float)w[e], qs[8 * c + e], dot);
-            }
-            s = dot * a.scale + m;
-        }
-        const float mc = wave_max_f(s);
-        if (mc == -INFINITY && !__any(s != s)) continue;  // uniform: nothing of the chunk is seen
-        const float Mn = fmaxf(M, mc), r = M == Mn ? 1.0f : expf(M - Mn), p = expf(s - Mn);
-        S = S * r + wave_sum_f(s == -INFINITY ? 0.0f : p);
-        M = Mn;
-        own();
-        ps[lane] = s == -INFINITY ? -1.0f : p;
-        own();
-#pragma unroll
-        for (int c = 0; c < DL; c++) acc[c] *= r;
-#pragma unroll 1
-        for (int t0 = 0; t0 < 64; t0 += NV) {
-            _Float16 v[NV][DL];
-#pragma unroll
-            for (int t = 0; t < NV; t++)
-#pragma unroll
-                for (int c = 0; c < DL; c++)
-                    v[t][c] = ((const _Float16 *)(vb + min(base + t0 + t, j1 - 1) * a.v_nb1))[64 * c + lane];
-#pragma unroll
-            for (int t = 0; t < NV; t++) {
-                const float pt = ps[t0 + t];
-#pragma unroll
-                for (int c = 0; c < DL; c++) acc[c] = pt < 0.0f ? acc[c] : fmaf(pt, (float)v[t][c], acc[c]);
-            }
-        }
-    }
-    const float inv = a.nsplit > 1 ? 1.0f : (S == 0.0f ? 0.0f : 1.0f / S);
-    float *part = a.part + ((i * a.n_head + h) * a.nsplit + split) * (D + 2);
-    float *o = a.nsplit > 1 ? part + 2 : a.dst + (i * a.n_head + h) * D;
-#pragma unroll
-    for (int c = 0; c < DL; c++) o[64 * c + lane] = acc[c] * inv;
-    if (a.nsplit > 1 && lane == 0) {
-        part[0] = M;
-        part[1] = S;
-    }
-}
-
 template <int D, bool MASK>
 __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
     using L = FmLds<D>;
@@ -447,11 +379,13 @@ bool fa_mfma_supported(const FaArgs &a) {
            (a.n_q * a.gqa + FM_P - 1) / FM_P <= 65535;
 }
 
-// Splits of the positions: toward 256 workgroups (one to a CU), each of at least FM_W steps.
+// Splits of the positions: toward 256 workgroups (one to a CU), each of at least FM_W steps; none where the merge's launch
+// costs more than further turns (us, one split / one turn a split: 5 rows at 320 positions, 16 heads on 8 of 128 8.6 /
+// 10.0, 16 of 64 6.8 / 9.1; at 1088 12.0 / 10.3 in splits of two turns).
 void fa_mfma_split(FaArgs &a) {
     const int64_t units = a.n_head / a.gqa * ((a.n_q * a.gqa + FM_P - 1) / FM_P), turn = FM_W * FM_STEP;
     const int64_t turns = (a.n_kv + turn - 1) / turn;
-    int64_t want = units >= 160 ? 1 : 256 / units;
+    int64_t want = units >= 160 || turns <= (a.D == 64 ? 3 : 2) ? 1 : 256 / units;
     want = want > turns ? turns : (want > 64 ? 64 : want);  // the merge holds one split per lane
     const int64_t per = (turns + want - 1) / want;
     a.nsplit = (int)((turns + per - 1) / per);

@@ -547,6 +547,9 @@ __device__ __forceinline__ float fa_mask_value(const FaStage &st, const uint16_t
 // position p (the last split when p lies past the positions read) turns kv head hk's key, stores key and value into
 // the caches at row p and stages them from LDS in place of that row's (not yet written) cache bytes. No other
 // workgroup reads row p, so the stores race with nothing.
+//
+// Of several rows (fa_rows_kernel), masks may hide positions that hold infinities or NaN (0 times them is NaN): sums that
+// are not finite are then formed again over the positions that the row sees, as k_fa_mfma does.
 template <int G, bool POST>
 __global__ __launch_bounds__(256) void k_fa_gqa(FaArgs a, QkvPostArgs pa) {
     constexpr int D = 128, T = 256 / (G * 64), CPT = D / T, PP = 256 / G / 64, PLEN = 64 / PP;
@@ -701,7 +704,7 @@ __global__ __launch_bounds__(256) void k_fa_gqa(FaArgs a, QkvPostArgs pa) {
             const float mc = wave_max_f(sv);
             const float Mold = hm[wave];
             float r = 1.0f, p = 0.0f, Mn = Mold;
-            if (mc != -INFINITY) {
+            if (mc != -INFINITY || (!POST && __any(sv != sv))) {
                 Mn = fmaxf(Mold, mc);
                 r = expf(Mold - Mn);
                 p = sv == -INFINITY ? 0.0f : expf(sv - Mn);
@@ -734,11 +737,13 @@ __global__ __launch_bounds__(256) void k_fa_gqa(FaArgs a, QkvPostArgs pa) {
     accs[(part_v * G + g_v) * D + 2 * cp] = acc0;
     accs[(part_v * G + g_v) * D + 2 * cp + 1] = acc1;
     __syncthreads();
+    bool odd = false;  // a sum that is not finite
     for (int e = tid; e < G * D; e += 256) {
         const int g = e / D, c = e % D;
         float tot = 0.0f;
 #pragma unroll
         for (int pp = 0; pp < PP; pp++) tot += accs[(pp * G + g) * D + c];
+        odd |= !(fabsf(tot) < INFINITY);
         const int64_t h = hk * G + g;
         if (a.nsplit == 1) {
             const float S = hs[g];
@@ -751,6 +756,10 @@ __global__ __launch_bounds__(256) void k_fa_gqa(FaArgs a, QkvPostArgs pa) {
                 part[1] = hs[g];
             }
         }
+    }
+    if constexpr (!POST) {
+        if (a.n_q == 1 || !__syncthreads_or(odd)) return;  // (it also orders the stores above before those below)
+        if (wave < G) fa_row_alone<D>(a, split, hk * G + wave, i, lane, qs[wave], ps[wave]);
     }
 }
 
@@ -850,6 +859,23 @@ int fa_splits(int64_t n_q, int64_t n_head, int64_t n_kv, int64_t gqa, int D) {
     want = want > 64 ? 64 : want;  // the merge holds one split per lane
     const int64_t per = (blocks + want - 1) / want;  // blocks per split
     return (int)((blocks + per - 1) / per);
+}
+
+// Whether a call of several rows is faster here than on the matrix cores (k_fa_mfma), which take 6.5 us for one step of the
+// smallest call, 8.6 for the second 256 positions and about 10 from the third on, the splits' merge included. Here a
+// chunk of 64 positions of one row and kv head is a workgroup's work, so that up to 256 of them (C below) are one round:
+// 4.6 us where one chunk is all there is (no merge), 7 to 8 with the merge. us, here / there, 16 heads on 8 of 128:
+// 10 rows at 64 positions 4.7 / 7.1, 64 rows 5.6 / 7.3, 128 rows 8.3 / 7.3; at 128 (C = 160) 7.6 / 7.2; at 320 six rows 7.3 /
+// 8.7, eight 9.3 / 8.7; at 512 eight rows 9.1 / 9.7, ten 10.4 / 10.1; at 1088 three rows 9.0 / 9.9, four 11.1 / 9.9.
+// One head to a kv head takes least, four most: 16 on 16, 64 rows at 64 positions 6.0 / 7.3; 32 on 8, four rows at 576
+// 10.5 / 9.9.
+bool fa_rows_kernel(const FaArgs &a) {
+    if (!fa_grouped(a.D, a.gqa)) return false;
+    const int64_t blocks = (a.n_kv + 63) / 64, units = a.n_q * (a.n_head / a.gqa), C = units * blocks;
+    if (blocks * a.gqa <= 4 && blocks <= 3 && fa_splits(a.n_q, a.n_head, a.n_kv, a.gqa, a.D) == 1)
+        return C <= (a.gqa == 1 ? 1024 : 512);
+    if (a.gqa == 4) return blocks >= 5 && C <= 256;
+    return blocks >= 3 && C <= (blocks < 8 ? 256 : 512);
 }
 
 hipError_t launch_fa_merge(const FaArgs &a, hipStream_t s) {

@@ -1258,7 +1258,8 @@ MX_API int mx_supports_flash_attn_ext(const mx_tensor *q, const mx_tensor *k, co
 }
 
 // Validation, arguments and scratch of an attention launch (mx_flash_attn_ext; mx_attn_decode). *mfma (when given)
-// becomes true for a call that goes to the matrix cores: several rows, and the scratch of its splits can be had.
+// becomes true for a call that goes to the matrix cores: several rows, not so few that the one-row kernel is faster, and
+// the scratch of its splits can be had.
 static int fa_args(mx_backend *be, const mx_tensor *q, const mx_tensor *k, const mx_tensor *v, const mx_tensor *mask,
                    const mx_tensor *dst, float scale, mx::FaArgs *a, bool *mfma = nullptr) {
     if (!mx_supports_flash_attn_ext(q, k, v, mask, dst, 0.0f, 0.0f))
@@ -1284,16 +1285,27 @@ static int fa_args(mx_backend *be, const mx_tensor *q, const mx_tensor *k, const
     auto part_bytes = [&]() {
         return (size_t)a->n_q * (size_t)a->n_head * (size_t)a->nsplit * (size_t)(a->D + 2) * 4;
     };
+    auto rows_split = [&]() {
+        a->nsplit = mx::fa_splits(a->n_q, a->n_head, a->n_kv, a->gqa, a->D);
+        a->split_len = ((a->n_kv + 63) / 64 + a->nsplit - 1) / a->nsplit * 64;  // whole 64-position blocks per split
+    };
+    auto room = [&]() {
+        if (a->nsplit > 1 && !ensure_work(be, part_bytes())) return false;
+        a->part = (float *)be->work;
+        return true;
+    };
+    if (mfma && mx::fa_rows_kernel(*a)) {
+        rows_split();
+        if (room()) return MX_SUCCESS;
+    }
     if (mfma && mx::fa_mfma_supported(*a)) {
         mx::fa_mfma_split(*a);
-        if (a->nsplit == 1 || ensure_work(be, part_bytes())) {
-            a->part = (float *)be->work;
+        if (room()) {
             *mfma = true;
             return MX_SUCCESS;
         }
     }
-    a->nsplit = mx::fa_splits(a->n_q, a->n_head, a->n_kv, a->gqa, a->D);
-    a->split_len = ((a->n_kv + 63) / 64 + a->nsplit - 1) / a->nsplit * 64;  // whole 64-position blocks per split
+    rows_split();
     if (a->nsplit > 1) {
         int rc = ensure_scratch(be, part_bytes());
         if (rc) return rc;

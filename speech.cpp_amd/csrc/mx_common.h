@@ -360,6 +360,8 @@ hipError_t launch_fa_merge(const FaArgs &a, hipStream_t s);
 // Several query rows on the matrix cores (attn.hip): whether it takes the call, the splits it takes (a.nsplit,
 // a.split_len; nsplit > 1 needs a.part as above), the launch.
 bool fa_mfma_supported(const FaArgs &a);
+// ... and whether the one-row kernel is faster for a few rows over few positions (layer.hip).
+bool fa_rows_kernel(const FaArgs &a);
 void fa_mfma_split(FaArgs &a);
 hipError_t launch_fa_mfma(const FaArgs &a, hipStream_t s);
 // One decode row: launch_qkv_post and launch_flash_attn in one attention launch (head size 128, gqa 1, 2 or 4; the

@@ -153,6 +153,63 @@ def test_hidden_odd_values(mx, be, heads, kv, D, odd):
     assert ok[:3].all() and np.all(np.abs(got[ok] - want[ok]) <= np.broadcast_to(bound, want.shape)[ok])
 
 
+@pytest.mark.parametrize("odd", ["nan", "inf", "key"])
+@pytest.mark.parametrize("rows,n_kv", [(4, 500), (7, 300), (20, 60)])
+@pytest.mark.parametrize("heads,kv", [(3, 3), (4, 2), (8, 2)])
+def test_hidden_odd_values_few_rows(mx, be, heads, kv, rows, n_kv, odd):
+    """The same where a few rows go to the one-row kernel; a row that sees nothing but a NaN score is NaN."""
+    past = n_kv - rows - 8
+    q, k, v, mask = case(rows, n_kv, heads, kv, 128, 6, past)
+    mask[0, 17] = -np.inf
+    want, bound = exact(q, k, v, mask, 0.1)
+    at = [17, past + rows - 1, past + rows + 3]  # hidden from the first row, from all but the last, from all
+    for j in at:
+        (k if odd == "key" else v)[j, :, ::3] = np.nan if odd == "key" else float(odd)
+    got = device(mx, be, q, k, v, mask, 0.1, cap=n_kv + 8)
+    assert np.all(np.abs(got[0] - want[0]) <= np.broadcast_to(bound, want.shape)[0])
+    if odd == "key":
+        assert np.isnan(got[1:]).all()
+        mask[2] = -np.inf
+        mask[2, 17] = 0
+        assert np.isnan(device(mx, be, q, k, v, mask, 0.1)[2]).all()
+    else:
+        assert not np.isfinite(got[1:, :, ::3]).any()
+        assert np.all(np.abs(got - want) <= bound, where=(np.arange(128) % 3 != 0))
+
+
+# either side of the lines between the kernels: one chunk of 64, two, three, eight (64-position chunks of 512 and 256 in all)
+@pytest.mark.parametrize("rows,n_kv,heads,kv", [(64, 64, 16, 8), (65, 64, 16, 8), (64, 64, 16, 16), (65, 64, 16, 16),
+                                                (32, 128, 16, 8), (8, 256, 16, 8), (9, 256, 16, 8), (8, 449, 16, 8),
+                                                (9, 449, 16, 8), (6, 300, 32, 8), (7, 300, 32, 8), (128, 192, 2, 2)])
+def test_kernel_lines(mx, be, rows, n_kv, heads, kv):
+    q, k, v, mask = case(rows, n_kv, heads, kv, 128, rows, n_kv - rows)
+    want, bound = exact(q, k, v, mask, 0.088)
+    assert np.all(np.abs(device(mx, be, q, k, v, mask, 0.088, mask_pad=(-n_kv) % 8) - want) <= bound)
+
+
+def test_few_rows_recorded_without_scratch(mx):
+    """A call that the one-row kernel would take in splits, recorded with no eager run before it: no scratch to be had, so
+    the matrix cores take it in one."""
+    be = mx.Backend(0)
+    rows, n_kv, heads, kv, D = 3, 250, 4, 2, 128
+    q, k, v, _ = case(rows, n_kv, heads, kv, D, 2)
+    want, bound = exact(q, k, v, None, 0.09)
+    K, V = (be.tensor(mx.F16, (kv * D, n_kv), x.reshape(n_kv, -1).view(np.uint16)) for x in (k, v))
+    Q, Y = be.tensor(mx.F32, (heads * D, rows), q.reshape(rows, -1)), be.tensor(mx.F32, (D, heads, rows))
+    views = [c.view((D, n_kv, kv), (2, kv * D * 2, D * 2)) for c in (K, V)]
+    be.graph_begin()
+    be.flash_attn_ext(Q.view((D, rows, heads), (4, heads * D * 4, D * 4)), views[0], views[1], None, Y, 0.09)
+    g = be.graph_end()
+    for _ in range(3):
+        Y.set(np.zeros((rows, heads, D), np.float32))
+        be.graph_launch(g)
+        be.sync()
+        assert np.all(np.abs(Y.numpy().reshape(rows, heads, D) - want) <= bound)
+    be.graph_free(g)
+    del Q, K, V, Y, views
+    be.close()
+
+
 @pytest.mark.parametrize("heads,kv,D", [(8, 1, 128), (12, 4, 128), (8, 1, 64), (16, 16, 64)])
 def test_weights_in_full(mx, be, heads, kv, D):
     """Scores that are exact in fp32 (one product each), so that the error is the weights' own and that of their sums. A
