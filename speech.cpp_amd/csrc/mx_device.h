@@ -157,10 +157,11 @@ __device__ __forceinline__ int pack4(int a, int b, int c, int d) {
 
 // ------------------------------------------------------------------------------------------------------------------
 // Correctly rounded quotients for the quantizers, without the scaling steps of a general division (Markstein's corrected
-// quotient: q = a r, q + r (a - b q)), and without a branch to one: the code of a general division that is never
-// reached still costs a decode step 25 us in 680, its instructions being fetched in 140 short kernels. The divisor's
-// mantissa is divided by and the exponent put back, which is exact while the quotient is normal or overflows. Each was
-// compared with the IEEE division over every finite or infinite float of its range on this chip.
+// quotient: q = a r, q + r (a - b q)). The Q8_0 / Q8_1 quantizer has no branch to a general division either: its code,
+// even when never reached, costs a decode step 25 us in 680, its instructions being fetched in 140 short kernels
+// (quant256_wave keeps one, for a scale whose reciprocal may be subnormal). The divisor's mantissa is divided by and the
+// exponent put back, which is exact while the quotient is normal or overflows. v_rcp_f32's last bit is the chip's own, so
+// that a correct rounding is a matter of measurement: the tests quantize blocks of every mantissa.
 // ------------------------------------------------------------------------------------------------------------------
 __device__ __forceinline__ bool mid_range(float v) {  // |v| in [2^-60, 2^60)
     return (__float_as_uint(v) & 0x7FFFFFFFu) - (67u << 23) < (120u << 23);

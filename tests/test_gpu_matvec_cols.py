@@ -97,3 +97,83 @@ def test_quantizers_over_all_exponents(mx, be, qt, rounding):
     got = out.get_bytes()[: O.row_size(qt, K) * len(es)].reshape(len(es), -1)
     want = O.quantize_rows(qt, x, rounding)
     assert np.array_equal(got, want), f"rows differing: {es[(got != want).any(axis=1)]}"
+
+
+def q8_blocks(x, rounding):
+    """Blocks [n, 32] as the device quantizes them, with IEEE divisions: d (fp16) and codes. Casts to int saturate, NaN is 0
+    (the C source leaves those to the machine)."""
+    f = np.float32
+    with np.errstate(all="ignore"):
+        a = np.abs(x).max(1, keepdims=True)
+        d = a / f(127)
+        if rounding == O.ROUND_X86:
+            q = np.rint(x * np.where(a != 0, f(127) / a, f(0)))
+        else:
+            v = x * np.where(d != 0, f(1) / d, f(0))  # roundf: half away from zero, exact in double
+            q = np.where(np.isfinite(v), np.copysign(np.floor(np.abs(v).astype(np.float64) + 0.5), v), v)
+        q = np.nan_to_num(q.astype(np.float64), nan=0, posinf=2.0 ** 31 - 1, neginf=-2.0 ** 31)
+        return d[:, 0].astype(np.float16), np.clip(q, -2.0 ** 31, 2.0 ** 31 - 1).astype(np.int64).astype(np.int8)
+
+
+def q8_device(mx, be, x, rounding):
+    out = be.quantize_act(O.TYPE_Q8_0, rounding, be.tensor(mx.F32, (x.size,), x), x.size, 1)
+    be.sync()
+    b = out.get_bytes()[:34 * len(x)].reshape(-1, 34)
+    return b[:, :2].copy().view(np.float16)[:, 0], b[:, 2:].view(np.int8)
+
+
+ROUNDINGS = pytest.mark.parametrize("rounding", [O.ROUND_REF, O.ROUND_X86], ids=["ref", "x86"])
+
+
+@ROUNDINGS
+def test_q8_0_over_every_mantissa(mx, be, rounding):
+    """A block for each float of [1, 2) as its largest, the others near the halves between codes: there the last bit of the
+    reciprocal shows."""
+    n = 1 << 20
+    half = (np.arange(32) * 4 % 127 + 0.5).astype(np.float32) / np.float32(127) * np.where(np.arange(32) % 2, -1, 1).astype(np.float32)
+    half[0] = 1
+    for part in range(8):
+        v = (np.arange(n, dtype=np.uint32) + np.uint32(0x3F800000 + part * n)).view(np.float32)
+        x = v[:, None] * half
+        d, q = q8_device(mx, be, x, rounding)
+        want_d, want_q = q8_blocks(x, rounding)
+        assert np.array_equal(d.view(np.uint16), want_d.view(np.uint16)) and np.array_equal(q, want_q)
+
+
+@ROUNDINGS
+def test_q8_0_at_the_ends(mx, be, rounding):
+    """Zero blocks, subnormal maxima (whose reciprocal overflows, and past that), mantissas of all ones and of one bit at
+    every exponent, the largest float, infinities."""
+    g = np.random.default_rng(3)
+    e = np.arange(0, 255, dtype=np.uint32) << 23
+    top = np.concatenate([np.arange(1, 300, dtype=np.uint32), 1 << np.arange(23, dtype=np.uint32), e, e + 1, e + 0x7FFFFF, e + 0x400000,
+                          np.array([0, 0x7F7FFFFF, 0x7F800000, 0x7F800000], np.uint32)]).view(np.float32)
+    x = (g.uniform(-1, 1, (len(top), 32)) * np.where(np.isfinite(top), top, 1)[:, None]).astype(np.float32)
+    x[np.arange(len(top)), g.integers(0, 32, len(top))] = top * g.choice([-1, 1], len(top)).astype(np.float32)
+    x[0] *= -0.0
+    d, q = q8_device(mx, be, x, rounding)
+    want_d, want_q = q8_blocks(x, rounding)
+    assert np.array_equal(d.view(np.uint16), want_d.view(np.uint16))
+    assert np.array_equal(q, want_q), top[(q != want_q).any(1)]
+
+
+def test_q8_k_over_every_mantissa(mx, be):
+    """d = 1 / (-127 / largest) of Q8_K blocks, fp32, for each float of [1, 2) and, at every exponent, a few mantissas. The
+    blocks overlap: rows of 256 floats, 16 bytes apart, of values that descend, each block's first its largest."""
+    def check(v):  # descending
+        x = np.zeros(4 * len(v) + 256, np.float32)
+        x[:4 * len(v):4] = v
+        X = be.tensor(mx.F32, (x.size,), x)
+        X.desc.nb[1] = 16
+        out = be.quantize_act(O.TYPE_Q8_K, O.ROUND_REF, X, 256, len(v))
+        be.sync()
+        d = out.get_bytes()[:292 * len(v)].reshape(-1, 292)[:, :4].copy().view(np.float32)[:, 0]
+        with np.errstate(all="ignore"):
+            want = np.float32(1) / (np.float32(-127) / v)
+        assert np.array_equal(d.view(np.uint32), want.view(np.uint32)), v[d.view(np.uint32) != want.view(np.uint32)]
+
+    for top in range(0x3FFFFFFF, 0x3F7FFFFF, -65535):  # (rows are grid.y)
+        check(np.arange(top, max(top - 65535, 0x3F7FFFFF), -1, dtype=np.uint32).view(np.float32))
+    m = np.array([0, 1, 2, 3, 0x2AAAAA, 0x3FFFFF, 0x400000, 0x555555, 0x7FFFFD, 0x7FFFFE, 0x7FFFFF], np.uint32)
+    all_e = np.sort(np.concatenate([(np.arange(0, 255, dtype=np.uint32)[:, None] << np.uint32(23) | m).ravel(), [0x7F800000]]))
+    check(all_e[1:][::-1].astype(np.uint32).view(np.float32).copy())
