@@ -31,7 +31,7 @@ constexpr int KS = 128;       // K per LDS stage
 // allocated for. What bounds both tiles is the VALU's conversion and fma per element and block (63% of the cycles at
 // M = 512, gate and up of 2 x 6144 rows, K = 2048; the matrix cores 22%), so its other instructions are kept few: 32-bit
 // index arithmetic, LDS offsets as immediates, scales of the idle lanes read as zeros instead of selected.
-// 64 x 64: three stages (54 KB, three workgroups per CU), block kb + 1's MFMAs issued before block kb's VALU. Against
+// 64 x 64: three stages (52 KB, three workgroups per CU), block kb + 1's MFMAs issued before block kb's VALU. Against
 // four stages, two workgroups and 64-bit indexes: q / k / v of K = 2048 at M = 512 22.5 -> 21.5 us, gate and up at M = 130
 // 27.2 -> 23.2, down (K = 6144, N = 2048) at M = 512 36.3 -> 32.6.
 // 64 x 128: two stages (52 KB) and one block at a time, so three workgroups share a CU: 43.1 us at M = 512 on gate and
@@ -119,7 +119,8 @@ struct I8Lds {
     static constexpr int QA = BM / 32, QB = BN / 32, NDX = BM / 32, NSC = (BM + BN) / 32, QS = (NSC + 3) / 4;
     static constexpr int OPS = QA + QB + QS;
     static_assert(SIZE <= 80 * 1024 || (BM == 128 && BN == 128), "two workgroups per CU");
-    static_assert(NS >= 2 && NS <= 4, "a ring of two to four stages");
+    static_assert(NS == 2 || NS == 3, "the waits of the stage loop");
+    static_assert(BM != 64 || BN != 64 || NS == 3, "the stage loop's slots");
 };
 
 __device__ __forceinline__ uint32_t i8_swz(uint32_t r) { return (r >> 1) & 7; }
@@ -255,7 +256,6 @@ k_gemm_q8_0_i8(GemmArgs a) {
         // instruction: __syncthreads' release fence would wait for the copies still in flight too.
         const int rem = nloc - 1 - s;  // stages issued after s: min(rem, NS - 2)
         if (rem >= L::NS - 2) wait_vm<(L::NS - 2) * L::OPS>();
-        else if (L::NS > 3 && rem == 1) wait_vm<L::OPS>();
         else wait_vm<0>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (s + L::NS - 1 < nloc) dma.issue(lds, (slot + L::NS - 1) % L::NS, kb0 + (s + L::NS - 1) * KS);

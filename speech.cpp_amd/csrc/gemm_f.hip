@@ -101,7 +101,7 @@ struct FgCfg {
     // Sums of sums: see the kernel. Three levels where the accumulators are few.
     static constexpr bool MID = TM * TN * NR <= 32;
     static_assert(NW <= 8 && KG * (CA + CB) % NW == 0 && WM % T == 0 && WN % T == 0, "tile");
-    static_assert(LDS <= 160 * 1024 && NS >= 2, "LDS");
+    static_assert(LDS <= 160 * 1024 && (NS == 2 || NS == 3), "LDS, and the waits of a stage");
     static_assert((KG - 1) * WGM * WGN * TM * TN * NR * 256 <= LDS, "the groups' sums fit the ring");
 };
 
@@ -221,7 +221,6 @@ __global__ __launch_bounds__(64 * C::NW) void k_gemm_f(FgArgs a) {
         // copies overwrite (the bare barrier: __syncthreads would wait for the copies in flight too)
         const int rem = nst - 1 - s;
         if (rem >= C::NS - 2) wait_vm<(C::NS - 2) * C::OPS>();
-        else if (C::NS > 3 && rem == 1) wait_vm<C::OPS>();
         else wait_vm<0>();
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (s + C::NS - 1 < nst) issue((s + C::NS - 1) % C::NS, st0 + s + C::NS - 1);
