@@ -137,7 +137,8 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
         issue_v(wave);
     }
     // the pairs' q rows, rounded to fp16 as ggml converts q to K's type: one 8-channel chunk per thread, through LDS (each
-    // lane reading its fragments from its own row costs 64 lines a load)
+    // lane reading its fragments from its own row costs 64 lines a load). Loads return in order, so a wave that waits for
+    // its q has its first step's copies too.
     if (tid < FM_P * L::CH) {
         const int pr = tid / L::CH, c = tid % L::CH;
         const uint32_t pc = min(p0 + (uint32_t)pr, np - 1), qi = pc / gqa;
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(64 * FM_W) void k_fa_mfma(FaArgs a) {
     for (int kb = 0; kb < KB; kb++) ko[kb] = (uint32_t)(L::K + fr * L::RB + 16 * ((2 * kb + fh) ^ fm_swk<D>(fr)));
     // B fragments of S^T: column (pair) fr, k = 16 kb + 8 fh ..
     v8h qf[KB];
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the copies stay in flight)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
     for (int kb = 0; kb < KB; kb++) qf[kb] = *(const v8h *)(smem + L::Q + ko[kb]);
     // a transposed read gives lane l of each 16 the four rows (4 fh ..) of value channel l; rows 8 u + 4 fh .. + 3
