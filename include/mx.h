@@ -320,6 +320,12 @@ MX_API int mx_peak_mfma(mx_backend *be, int kind, int workgroups, int iters);
  * backend's scratch: once a later op grows the scratch (and frees the old one), mx_graph_launch refuses every graph
  * recorded before that with MX_FAILED, and the caller records it again. A graph launches only on the backend that
  * recorded it (MX_INVALID otherwise).
+ * Two ops use scratch that a backend keeps apart, and that no graph is refused for: MUL_MAT of more than 8 columns on
+ * F16 / F32 weights (64 MB, or what one batch slice takes), and FLASH_ATTN_EXT of several rows (up to 5 MB). It grows at
+ * least twofold, and buffers that it outgrew are freed with the backend only, so graphs recorded on them stay
+ * valid. Recorded without an eager run before, while it is too small, these ops take the form that needs none, for as long
+ * as the graph lives: other sums to the same precision, and slower (the product eight columns at a time: 2,600 us instead
+ * of 39 for 512 rows of F16 12288 x 2048). Attention that every form would split is refused, as any op without its scratch.
  * ------------------------------------------------------------------------------------------------------------- */
 MX_API int mx_graph_begin(mx_backend *be);
 MX_API int mx_graph_end(mx_backend *be, mx_graph **graph);
