@@ -17,8 +17,9 @@
 // (geometric) average; with exact scores, few positions: 7.3e-8 against 7.7e-8.
 //
 // What bounds it: the VALU, at about 14 issue slots a score against 6 of the matrix cores (two waves per SIMD). 512 rows
-// at 1024 positions before them, 16 heads on 8 of 128: 19.4 us (four waves and a two-slot ring 29.6; q not staged through LDS and the rescale
-// inside the loop 25.5); one workgroup per row (k_fa_gqa), with the q / k norms, RoPE and stores before it, 365.
+// at 1024 positions before them, 16 heads on 8 of 128: 21 us, 25 with the q / k norms, RoPE and stores before it, where
+// one workgroup per row (k_fa_gqa) takes 366 (an earlier form 16-21 us; on four waves and a two-slot ring 29.6, q not
+// staged through LDS and the rescale inside the loop 25.5).
 #include "mx_common.h"
 #include "mx_device.h"
 
