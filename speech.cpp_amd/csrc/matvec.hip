@@ -459,7 +459,7 @@ static hipError_t launch_nc(const MatvecArgs &a, int64_t maxN, size_t lds, hipSt
 }
 
 template <int TYPE>
-hipError_t launch_matvec_q(const MatvecArgs &a, int64_t maxN, hipStream_t s) {
+static hipError_t launch_type(const MatvecArgs &a, int64_t maxN, hipStream_t s) {
     const size_t lds = act_lds_bytes(TYPE, a.K, a.ncols);
     switch (a.ncols) {
         case 1: return launch_nc<TYPE, 1>(a, maxN, lds, s);
@@ -474,6 +474,18 @@ hipError_t launch_matvec_q(const MatvecArgs &a, int64_t maxN, hipStream_t s) {
     }
 }
 
-template hipError_t launch_matvec_q<MX_MV_TYPE>(const MatvecArgs &a, int64_t maxN, hipStream_t s);
+hipError_t launch_matvec(const MatvecArgs &a, hipStream_t s) {
+    int64_t maxN = 0;
+    for (int i = 0; i < a.nprob; i++) maxN = a.prob[i].N > maxN ? a.prob[i].N : maxN;
+    if (maxN == 0) return hipSuccess;
+    if (a.type == MX_TYPE_F16 || a.type == MX_TYPE_F32) return launch_matvec_f(a, s);
+    switch (a.type) {
+        case MX_TYPE_Q8_0: return launch_type<MX_TYPE_Q8_0>(a, maxN, s);
+        case MX_TYPE_Q4_K: return launch_type<MX_TYPE_Q4_K>(a, maxN, s);
+        case MX_TYPE_Q5_K: return launch_type<MX_TYPE_Q5_K>(a, maxN, s);
+        case MX_TYPE_Q6_K: return launch_type<MX_TYPE_Q6_K>(a, maxN, s);
+        default: return hipErrorInvalidValue;
+    }
+}
 
 }  // namespace mx

@@ -166,19 +166,4 @@ hipError_t launch_matvec_f(const MatvecArgs &a, hipStream_t s) {
     }
 }
 
-hipError_t launch_matvec(const MatvecArgs &a, hipStream_t s) {
-    int64_t maxN = 0;
-    for (int i = 0; i < a.nprob; i++) maxN = a.prob[i].N > maxN ? a.prob[i].N : maxN;
-    if (maxN == 0) return hipSuccess;
-    switch (a.type) {
-        case MX_TYPE_F16:
-        case MX_TYPE_F32: return launch_matvec_f(a, s);
-        case MX_TYPE_Q8_0: return launch_matvec_q<MX_TYPE_Q8_0>(a, maxN, s);
-        case MX_TYPE_Q4_K: return launch_matvec_q<MX_TYPE_Q4_K>(a, maxN, s);
-        case MX_TYPE_Q5_K: return launch_matvec_q<MX_TYPE_Q5_K>(a, maxN, s);
-        case MX_TYPE_Q6_K: return launch_matvec_q<MX_TYPE_Q6_K>(a, maxN, s);
-        default: return hipErrorInvalidValue;
-    }
-}
-
 }  // namespace mx

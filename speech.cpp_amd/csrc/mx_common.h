@@ -195,9 +195,6 @@ struct MatvecArgs {
     int lpr;               // lanes per row forced (16, 32, 64), or 0 to pick by K
 };
 hipError_t launch_matvec(const MatvecArgs &a, hipStream_t s);
-// ... on one quantized type, maxN rows in the widest problem (matvec.hip, compiled once per type).
-template <int TYPE>
-hipError_t launch_matvec_q(const MatvecArgs &a, int64_t maxN, hipStream_t s);
 // The same products on F16 / F32 weights in ggml's row-major layout (prob[i].w.p0 = the weight's data; K % 8 == 0 for
 // F16, K % 4 == 0 for F32; no ids mode).
 hipError_t launch_matvec_f(const MatvecArgs &a, hipStream_t s);
