@@ -758,7 +758,9 @@ __global__ __launch_bounds__(256) void k_fa_gqa(FaArgs a, QkvPostArgs pa) {
         }
     }
     if constexpr (!POST) {
-        if (a.n_q == 1 || !__syncthreads_or(odd)) return;  // (it also orders the stores above before those below)
+        if (a.n_q == 1 || !__syncthreads_or(odd)) return;
+        wait_vm<0>();  // the stores above come first, whichever wave they are of
+        __syncthreads();
         if (wave < G) fa_row_alone<D>(a, split, hk * G + wave, i, lane, qs[wave], ps[wave]);
     }
 }
